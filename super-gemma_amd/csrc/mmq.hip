@@ -25,8 +25,17 @@
 //    costs the matrix cores less than the K=16 one: config 2 571 -> 620-627
 //    TOP/s, M = 4096 750 -> 786, with half the operand registers).  The VALU is
 //    left with one cvt and one FMA per output element and block, and that —
-//    not the MFMA — still bounds the kernel (a wave64 VALU op costs 4
-//    cycles against 32 for an MFMA covering 1024 elements).
+//    not the MFMA — bounds the kernel: a wave64 VALU op holds its SIMD for 4
+//    cycles, and counters put VALU issue at 93% of the cycles (M = 4096,
+//    K = 5376, N = 21504).  Every other VALU op of the loop therefore costs
+//    its share: with uniform pointers advanced by the scalar unit, one-op
+//    unpacks and the scale words moved up instead of selected, a stage takes
+//    632 VALU ops against 683 (512 of them cvt + FMA, 32 MFMA issues):
+//    1215-1221 -> 1146-1149 us there; K = 21504, M = 2048, split 4 666 -> 643;
+//    K = 5376, M = 512 172 -> 170.
+//  * Ragged tiles read clamped rows and run the same loop (they had a
+//    bounds-checked one: a 1500-token prompt of the released geometry
+//    15.3 -> 14.15 ms, M = 37, N = 8192 86 -> 81 us).
 //  * Tile order is XCD-aware: consecutive workgroup ids land on different
 //    XCDs (each with its own L2), so ids are remapped so that every XCD
 //    walks a contiguous range of N-tiles with all their M-tiles, and a
@@ -54,107 +63,94 @@ constexpr int kMWG = 256;
 
 struct Stage {
     int8_t a[BM * ROWB];      // activations, [row][k]
-    int8_t b[BN * ROWB];      // weights (q-8), [col][k]
-    uint16_t da[BM][KB];      // activation scales (f16 bits), [row][block]
-    uint16_t dw[BN][KB];      // weight scales (f16 bits), [col][block]
+    int8_t b[BN * ROWB];      // weights 16·(q-8), [col][k]
+    uint2 da[BM];             // activation scales (f16 bits), [row], 4 blocks
+    uint2 dw[BN];             // weight scales (f16 bits), [col], 4 blocks
+    uint2 zero[34];           // [0] and [32] zero: the scale words of lanes 32..63 (ld_scales)
 };
 
+// Nibbles as int8 16·(q-8): the nibble moved to the byte's high half with its
+// top bit flipped, one three-input logic op (plus a shift for the low
+// nibbles) per 4 weights against 3-4 for q-8 itself.  The factor 16 is taken
+// off the finished sums, exactly: a block dot stays below 2^20, and the sums
+// (scales are f16) far inside fp32's exponent range.
+constexpr float kUnscale = 1.0f / 16.0f;
 __device__ __forceinline__ uint32_t unpack_lo(uint32_t q) {
-    return ((q & 0x0F0F0F0Fu) + 0x78787878u) ^ 0x80808080u;  // nibble-8 as int8
+    return ((q << 4) & 0xF0F0F0F0u) ^ 0x80808080u;
 }
 __device__ __forceinline__ uint32_t unpack_hi(uint32_t q) {
-    return (((q >> 4) & 0x0F0F0F0Fu) + 0x78787878u) ^ 0x80808080u;
+    return (q & 0xF0F0F0F0u) ^ 0x80808080u;
 }
 
 struct Prefetch {
     v4i a[4];          // 64 activation bytes: row = tid/2, k-half = tid%2 (native
                        // vectors: HIP's uint4 is a struct, copied through scratch)
     uint32_t w[9];     // two Q4_0 blocks (36 bytes): col = tid/2, blocks 2*(tid%2)+{0,1}
-    uint16_t da[4];    // threads < 128: 4 block scales of row tid
+    uint2 da;          // threads < 128: 4 block scales of row tid
 };
 
-__device__ __forceinline__ void load_stage(Prefetch &pf, const int8_t *__restrict__ xq,
-                                           const uint16_t *__restrict__ xs,
-                                           const uint8_t *__restrict__ W, int m, int n, int k,
-                                           int nb, int m0, int n0, int b0, int b_end) {
-    const int t = threadIdx.x;
-    {   // activations: 64 contiguous bytes
-        const int row = t >> 1, half = t & 1;
-        const int gm = m0 + row;
-        const int kb = b0 * 32 + half * 64;  // first K index of this thread's 64 bytes
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int kk = kb + i * 16;
-            if (gm < m && kk < b_end * 32)
-                pf.a[i] = *reinterpret_cast<const v4i *>(xq + (size_t)gm * k + kk);
-            else
-                pf.a[i] = v4i{0, 0, 0, 0};
-        }
-    }
-    {   // weights: two blocks, 36 bytes, 4-aligned (b0 and the pair index are even)
-        const int col = t >> 1, pair = t & 1;
-        const int gn = n0 + col;
-        const int b = b0 + 2 * pair;
-        if (gn < n && b < b_end) {
-            const uint32_t *src =
-                reinterpret_cast<const uint32_t *>(W + ((size_t)gn * nb + b) * 18);
-            const bool two = b + 1 < b_end;
-#pragma unroll
-            for (int j = 0; j < 9; j++)
-                pf.w[j] = (j < 5 || two) ? src[j] : 0u;
-        } else {
-#pragma unroll
-            for (int j = 0; j < 9; j++) pf.w[j] = 0u;
-        }
-    }
-    if (t < BM) {
-        const int gm = m0 + t;
-#pragma unroll
-        for (int i = 0; i < KB; i++) {
-            const int b = b0 + i;
-            pf.da[i] = (gm < m && b < b_end) ? xs[(size_t)gm * nb + b] : (uint16_t)0;
-        }
-    }
-}
-
-// Aligned shapes (m % BM == 0, n % BN == 0, nb % KB == 0): no bounds
-// checks; each thread's three sources are base pointers that advance by a
-// constant per stage, and the 4 block scales of a row are one 8-byte load.
-struct AlignedSrc {
-    const int8_t *a;      // row t/2 of the tile, byte 64·(t%2) of block 0
-    const uint32_t *w;    // column t/2, block 2·(t%2)
-    const uint2 *da;      // row t (t < BM): scales of blocks 0..3
+// A tile's three sources: uniform pointers (scalar registers, advanced by
+// the scalar unit) plus a 32-bit offset per thread that stays fixed, so a
+// stage's loads cost the VALU nothing.  Rows past m and columns past n
+// (ragged tiles) read the last row / column instead, and their results are
+// not stored: odd sizes run the same loop as whole tiles.
+typedef const __attribute__((address_space(1))) char *gptr;
+template <typename O>         // uint32_t; uint64_t from kWideK on (128 rows' offsets)
+struct TileSrc {
+    gptr a, w, d;             // tile row 0 / column 0 / row 0, at the stage's first block
+    O oa, ow, od, od2;        // byte offsets: row t/2, byte 64·(t%2) / column t/2, block
+                              // 2·(t%2) / row t, blocks 0-1 and 2-3
 };
+constexpr uint32_t kWideK = 1u << 25;
 
-__device__ __forceinline__ AlignedSrc aligned_src(const int8_t *__restrict__ xq,
-                                                  const uint16_t *__restrict__ xs,
-                                                  const uint8_t *__restrict__ W, int k, int nb,
-                                                  int m0, int n0) {
-    const int t = threadIdx.x;
-    AlignedSrc s;
-    s.a = xq + (size_t)(m0 + (t >> 1)) * k + (t & 1) * 64;
-    s.w = reinterpret_cast<const uint32_t *>(W + ((size_t)(n0 + (t >> 1)) * nb + 2 * (t & 1)) * 18);
-    s.da = reinterpret_cast<const uint2 *>(xs + (size_t)(m0 + (t & (BM - 1))) * nb);
+template <typename O>
+__device__ __forceinline__ TileSrc<O> tile_src(const int8_t *__restrict__ xq,
+                                            const uint16_t *__restrict__ xs,
+                                            const uint8_t *__restrict__ W, int m, int n, int k,
+                                            int nb, int m0, int n0) {
+    const uint32_t t = threadIdx.x, pair = nb < KB ? 0 : t & 1;  // nb = 2: both read blocks 0-1
+    TileSrc<O> s;
+    s.a = (gptr)(xq + (size_t)m0 * k);
+    s.w = (gptr)(W + (size_t)n0 * nb * 18);
+    s.d = (gptr)(xs + (size_t)m0 * nb);
+    s.oa = (O)min((int)t >> 1, m - 1 - m0) * (O)k + pair * 64;
+    s.ow = ((O)min((int)t >> 1, n - 1 - n0) * (O)nb + 2 * pair) * 18;
+    s.od = (O)min((int)t & (BM - 1), m - 1 - m0) * (O)nb * 2;
+    s.od2 = s.od + (nb < KB ? 0 : 4);
     return s;
 }
 
-__device__ __forceinline__ void load_stage_al(Prefetch &pf, const AlignedSrc &src, int b0) {
-    const v4i *a = reinterpret_cast<const v4i *>(src.a + b0 * 32);
+typedef uint32_t u32a2 __attribute__((aligned(2)));  // xs is 2-byte aligned
+template <typename O>
+__device__ __forceinline__ void load_stage(Prefetch &pf, const TileSrc<O> &src, int b0) {
+    gptr a = src.a + (size_t)b0 * 32, w = src.w + (size_t)b0 * 18, d = src.d + (size_t)b0 * 2;
+    // Base in scalar registers, 32-bit offset in a vector register: the loads'
+    // own addressing form (the offsets are made opaque here, or the compiler
+    // widens them once outside the loop and adds 64-bit vectors per stage).
+    O oa = src.oa, ow = src.ow, od = src.od, od2 = src.od2;
+    asm volatile("" : "+s"(a), "+s"(w), "+s"(d), "+v"(oa), "+v"(ow), "+v"(od), "+v"(od2));
 #pragma unroll
-    for (int i = 0; i < 4; i++) pf.a[i] = a[i];
-    const uint32_t *w = src.w + (b0 * 18) / 4;  // b0 % 4 == 0: 72 B per stage
+    for (int i = 0; i < 4; i++)
+        pf.a[i] = *(const __attribute__((address_space(1))) v4i *)(a + oa + 16 * i);
     // plain loads: a weight strip serves every M-tile of its column group
     // (from L2); with the nontemporal hint config 2 ran at 526-530 against
     // 573-579 TOP/s and M = 4096 at 676 against 758-763
 #pragma unroll
-    for (int j = 0; j < 9; j++) pf.w[j] = w[j];
-    if (threadIdx.x < BM) {
-        const uint2 d = src.da[b0 / 4];
-        pf.da[0] = (uint16_t)(d.x & 0xffffu);
-        pf.da[1] = (uint16_t)(d.x >> 16);
-        pf.da[2] = (uint16_t)(d.y & 0xffffu);
-        pf.da[3] = (uint16_t)(d.y >> 16);
-    }
+    for (int j = 0; j < 9; j++)
+        pf.w[j] = *(const __attribute__((address_space(1))) uint32_t *)(w + ow + 4 * j);
+    if (threadIdx.x < BM)
+        pf.da = make_uint2(*(const __attribute__((address_space(1))) u32a2 *)(d + od),
+                           *(const __attribute__((address_space(1))) u32a2 *)(d + od2));
+}
+
+// Zero scales for the dead block pair of a K end with two blocks: their
+// products then add exact zeros (the dots are finite).
+__device__ __forceinline__ void kill_pair(Prefetch &pf, int dead) {
+    if ((int)(threadIdx.x & 1) == dead) pf.w[0] = pf.w[4] = 0u;
+    if (dead)
+        pf.da.y = 0u;
+    else
+        pf.da.x = 0u;
 }
 
 __device__ __forceinline__ void store_stage(const Prefetch &pf, Stage &S) {
@@ -185,13 +181,10 @@ __device__ __forceinline__ void store_stage(const Prefetch &pf, Stage &S) {
         *reinterpret_cast<uint4 *>(dst + 32) = lo;
         *reinterpret_cast<uint4 *>(dst + 48) = hi;
         // the two blocks' scales: low half of word 0, high half of word 4
-        *reinterpret_cast<uint32_t *>(&S.dw[col][2 * pair]) =
+        reinterpret_cast<uint32_t *>(&S.dw[col])[pair] =
             (pf.w[0] & 0xffffu) | (pf.w[4] & 0xffff0000u);
     }
-    if (t < BM) {
-#pragma unroll
-        for (int i = 0; i < KB; i++) S.da[t][i] = pf.da[i];
-    }
+    if (t < BM) S.da[t] = pf.da;
 }
 
 // Tile of the jl-th workgroup slot of XCD x (workgroup b runs on XCD b % 8,
@@ -239,7 +232,7 @@ struct TailSplit {
 // HOUT: the output is f16 (uint16_t bits, each sum rounded to nearest even:
 // the reference's y binding, gemm_q4_0_i8.wgsl:63); else fp32.  TAIL: the
 // tail split is built in (a separate kernel, so the others keep their code).
-template <bool AL, bool HOUT, bool TAIL = false>
+template <bool HOUT, bool TAIL = false, typename O = uint32_t>
 __global__ __launch_bounds__(kMWG, SGQ_MMQ_WG_PER_CU) void mmq_kernel(const uint8_t *__restrict__ W,
                                                       const int8_t *__restrict__ xq,
                                                       const uint16_t *__restrict__ xs,
@@ -289,17 +282,25 @@ __global__ __launch_bounds__(kMWG, SGQ_MMQ_WG_PER_CU) void mmq_kernel(const uint
     // flight while stage s computes (four blocks of MFMAs and rescales),
     // then go to the other LDS buffer
     Prefetch pf;
-    AlignedSrc src{};
-    if (AL) src = aligned_src(xq, xs, W, k, nb, m0, n0);
-    auto load = [&](Prefetch &p, int b0) {
-        if (AL)
-            load_stage_al(p, src, b0);
-        else
-            load_stage(p, xq, xs, W, m, n, k, nb, m0, n0, b0, b_end);
+    const TileSrc<O> src = tile_src<O>(xq, xs, W, m, n, k, nb, m0, n0);
+    // A range that ends with two blocks (nb is even, the split bounds are
+    // multiples of KB): its last stage starts two blocks early, with the scales
+    // of the pair it has seen zeroed, so its loads stay in the rows; a K of 64
+    // has one stage whose second pair is dead.
+    const bool short_end = (b_end - b_beg) % KB != 0;
+    const int dead = nb < KB ? 1 : 0;
+    auto load = [&](int s) {
+        const int b0 = b_beg + s * KB;
+        load_stage(pf, src, b0 + KB <= b_end || dead ? b0 : b_end - KB);
     };
+    auto store = [&](int s) {
+        if (short_end && s + 1 == n_stages) kill_pair(pf, dead);
+        store_stage(pf, stages[s & 1]);
+    };
+    if (threadIdx.x < 4) stages[threadIdx.x >> 1].zero[32 * (threadIdx.x & 1)] = make_uint2(0u, 0u);
     if (n_stages > 0) {
-        load(pf, b_beg);
-        store_stage(pf, stages[0]);
+        load(0);
+        store(0);
     }
     __syncthreads();
 
@@ -310,24 +311,28 @@ __global__ __launch_bounds__(kMWG, SGQ_MMQ_WG_PER_CU) void mmq_kernel(const uint
     };
     // the f16 scale bits of the wave's two row and two column tiles for the
     // stage's four blocks (two per word), read once per stage; zero in the
-    // lanes (h = 1) whose K terms of the scale MFMA are zero
-    uint2 sa4[2], sb4[2];
+    // lanes (h = 1) whose K terms of the scale MFMA are zero: they read the
+    // stage's zero words
+    uint32_t sa[2], sa2[2], sb[2], sb2[2];  // blocks 0-1, blocks 2-3
+    const uint32_t ga = (uint32_t)(h ? offsetof(Stage, zero) : offsetof(Stage, da) + (wm * 64 + r) * 8);
+    const uint32_t gb = (uint32_t)(h ? offsetof(Stage, zero) : offsetof(Stage, dw) + (wn * 64 + r) * 8);
     auto ld_scales = [&](const Stage &S) {
+        const uint8_t *sp = reinterpret_cast<const uint8_t *>(&S);
 #pragma unroll
         for (int i = 0; i < 2; i++) {
-            const uint2 a = *reinterpret_cast<const uint2 *>(&S.da[wm * 64 + i * 32 + r][0]);
-            const uint2 b = *reinterpret_cast<const uint2 *>(&S.dw[wn * 64 + i * 32 + r][0]);
-            sa4[i] = h == 0 ? a : make_uint2(0u, 0u);
-            sb4[i] = h == 0 ? b : make_uint2(0u, 0u);
+            const uint2 a = *reinterpret_cast<const uint2 *>(sp + ga + i * 256);
+            const uint2 b = *reinterpret_cast<const uint2 *>(sp + gb + i * 256);
+            sa[i] = a.x, sa2[i] = a.y, sb[i] = b.x, sb2[i] = b.y;
         }
     };
+    const uint32_t fa = (uint32_t)((wm * 64 + r) * ROWB + h * 16);
+    const uint32_t fb = (uint32_t)(offsetof(Stage, b) + (wn * 64 + r) * ROWB + h * 16);
     auto ld_ops = [&](const Stage &S, int blk, Ops &o) {
+        const uint8_t *sp = reinterpret_cast<const uint8_t *>(&S) + blk * 32;
 #pragma unroll
         for (int i = 0; i < 2; i++) {
-            o.af[i] = *reinterpret_cast<const v4i *>(
-                &S.a[(wm * 64 + i * 32 + r) * ROWB + blk * 32 + h * 16]);
-            o.bf[i] = *reinterpret_cast<const v4i *>(
-                &S.b[(wn * 64 + i * 32 + r) * ROWB + blk * 32 + h * 16]);
+            o.af[i] = *reinterpret_cast<const v4i *>(sp + fa + i * 32 * ROWB);
+            o.bf[i] = *reinterpret_cast<const v4i *>(sp + fb + i * 32 * ROWB);
         }
     };
     // Scale operands: lane (r, h = 0) holds K term 0 = d of its row (A) /
@@ -368,7 +373,7 @@ __global__ __launch_bounds__(kMWG, SGQ_MMQ_WG_PER_CU) void mmq_kernel(const uint
         }
     };
     auto step = [&](int s) {
-        if (s + 1 < n_stages) load(pf, b_beg + (s + 1) * KB);
+        if (s + 1 < n_stages) load(s + 1);
         const Stage &S = stages[s & 1];
         // the next block's LDS operands load while this block computes
         // (two blocks per iteration, so both operand sets keep fixed registers)
@@ -382,15 +387,15 @@ __global__ __launch_bounds__(kMWG, SGQ_MMQ_WG_PER_CU) void mmq_kernel(const uint
             uint32_t wa[2], wb[2];
 #pragma unroll
             for (int i = 0; i < 2; i++) {
-                wa[i] = bp == 0 ? sa4[i].x : sa4[i].y;
-                wb[i] = bp == 0 ? sb4[i].x : sb4[i].y;
+                wa[i] = sa[i], sa[i] = sa2[i];  // the next pair's word moves up
+                wb[i] = sb[i], sb[i] = sb2[i];
             }
             block(o0, wa, wb, false);
             ld_ops(S, min(bp + 2, KB - 1), o0);
             asm volatile("" ::: "memory");
             block(o1, wa, wb, true);
         }
-        if (s + 1 < n_stages) store_stage(pf, stages[(s + 1) & 1]);
+        if (s + 1 < n_stages) store(s + 1);
         __syncthreads();
     };
     for (int s = 0; s < n_stages; s++) step(s);
@@ -406,26 +411,33 @@ __global__ __launch_bounds__(kMWG, SGQ_MMQ_WG_PER_CU) void mmq_kernel(const uint
 #pragma unroll
                 for (int q = 0; q < 16; q++)
                     tp[(wm * 64 + i * 32 + 8 * (q / 4) + 4 * h + (q % 4)) * BN + wn * 64 + j * 32 +
-                       r] = acc[i][j][q];
+                       r] = acc[i][j][q] * kUnscale;
         return;
     }
+    auto put = [&](bool whole) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+        for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int col = n0 + wn * 64 + j * 32 + r;
-            if (!AL && col >= n) continue;
+            for (int j = 0; j < 2; j++) {
+                const int col = n0 + wn * 64 + j * 32 + r;
+                if (!whole && col >= n) continue;
 #pragma unroll
-            for (int q = 0; q < 16; q++) {
-                const int row = m0 + wm * 64 + i * 32 + 8 * (q / 4) + 4 * h + (q % 4);
-                if (AL || row < m) {
-                    if (HOUT)
-                        dsth[(size_t)row * n + col] = f32_to_f16_bits(acc[i][j][q]);
-                    else
-                        dst[(size_t)row * n + col] = acc[i][j][q];
+                for (int q = 0; q < 16; q++) {
+                    const int row = m0 + wm * 64 + i * 32 + 8 * (q / 4) + 4 * h + (q % 4);
+                    if (whole || row < m) {
+                        const float v = acc[i][j][q] * kUnscale;
+                        if (HOUT)
+                            dsth[(size_t)row * n + col] = f32_to_f16_bits(v);
+                        else
+                            dst[(size_t)row * n + col] = v;
+                    }
                 }
             }
-        }
+    };
+    if (m0 + BM <= m && n0 + BN <= n)
+        put(true);
+    else
+        put(false);
 }
 
 __global__ void splitk_reduce_kernel(const float4 *__restrict__ part, float4 *__restrict__ y,
@@ -447,7 +459,7 @@ __global__ void splitk_reduce_kernel(const float4 *__restrict__ part, float4 *__
 // y of the tail tiles: the tail_st parts summed in part order (float4 per
 // thread, one 128×128 tile per 16 workgroups of 256 threads).
 __global__ __launch_bounds__(256) void mmq_tail_reduce_kernel(TailSplit ts, float *__restrict__ y,
-                                                              int n, int mt, int nt) {
+                                                              int m, int n, int mt, int nt) {
     const int tiles = mt * nt, lx = tiles / kXcds - ts.fx;
     const int slot = blockIdx.x / 16;  // tail tile
     const int e = (blockIdx.x % 16) * 256 + threadIdx.x;  // float4 within the tile
@@ -464,6 +476,7 @@ __global__ __launch_bounds__(256) void mmq_tail_reduce_kernel(TailSplit ts, floa
         a.w += b.w;
     }
     const int row = e / (BN / 4), c4 = e % (BN / 4);
+    if (tm * BM + row >= m) return;
     *reinterpret_cast<float4 *>(y + (size_t)(tm * BM + row) * n + tn * BN + 4 * c4) = a;
 }
 
@@ -486,27 +499,24 @@ int gemm_t(hipStream_t st, const void *w, const int8_t *xq, const uint16_t *xs, 
     static bool attr = false;
     const size_t lds = 2 * sizeof(Stage);
     if (!attr) {
-        SGQ_HIP(hipFuncSetAttribute((const void *)mmq_kernel<false, HOUT>,
+        SGQ_HIP(hipFuncSetAttribute((const void *)mmq_kernel<HOUT>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        SGQ_HIP(hipFuncSetAttribute((const void *)mmq_kernel<true, HOUT>,
+        SGQ_HIP(hipFuncSetAttribute((const void *)mmq_kernel<HOUT, false, uint64_t>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        SGQ_HIP(hipFuncSetAttribute((const void *)mmq_kernel<true, false, true>,
+        SGQ_HIP(hipFuncSetAttribute((const void *)mmq_kernel<false, true>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         attr = true;
     }
     const int mt = (int)((m + BM - 1) / BM), nt = (int)((n + BN - 1) / BN);
     void *dst = split_k == 1 ? y : static_cast<void *>(partials);
-    // every split's block range is a multiple of KB when nb is (the split
-    // bounds are rounded down to KB)
-    const bool aligned = m % BM == 0 && n % BN == 0 && (k / 32) % KB == 0 &&
-                         ((uintptr_t)xs & 7) == 0;
-    // Tail split: aligned fp32 output, split_k = 1 and a partials buffer
-    // (m·n floats always suffice: the parts are at most one round of tiles)
+    // Tail split: fp32 output in whole column tiles, split_k = 1 and a
+    // partials buffer (m·n floats suffice when m is whole tiles; the parts are
+    // at most one round of tiles)
     TailSplit ts{0, 0, partials};
     const int tiles = mt * nt, slots_x = device_info().cus * SGQ_MMQ_WG_PER_CU / kXcds;
     // (only below two whole rounds: at M = 4096, N = 21504, with a tail of
     // half a round split in 2, the launch measured 1.3% slower)
-    if (aligned && !HOUT && split_k == 1 && partials != nullptr && tiles % kXcds == 0 &&
+    if (m % BM == 0 && n % BN == 0 && k < kWideK && !HOUT && split_k == 1 && partials != nullptr && tiles % kXcds == 0 &&
         slots_x > 0 && tiles / kXcds > slots_x && tiles / kXcds < 2 * slots_x) {
         const int tx = tiles / kXcds, fx = tx / slots_x * slots_x, lx = tx - fx;
         const int parts = lx > 0 ? std::min(4, slots_x / lx) : 0;
@@ -514,22 +524,22 @@ int gemm_t(hipStream_t st, const void *w, const int8_t *xq, const uint16_t *xs, 
     }
     const int grid_x = ts.st ? kXcds * (ts.fx + (tiles / kXcds - ts.fx) * ts.st) : tiles;
     if (ts.st)
-        hipLaunchKernelGGL((mmq_kernel<true, false, true>), dim3(grid_x, split_k), dim3(kMWG), lds,
-                           st, static_cast<const uint8_t *>(w), xq, xs, dst, (int)m, (int)n,
+        hipLaunchKernelGGL((mmq_kernel<false, true>), dim3(grid_x, split_k), dim3(kMWG), lds, st,
+                           static_cast<const uint8_t *>(w), xq, xs, dst, (int)m, (int)n, (int)k, mt,
+                           nt, (int)split_k, ts);
+    else if (k >= kWideK)
+        hipLaunchKernelGGL((mmq_kernel<HOUT, false, uint64_t>), dim3(grid_x, split_k), dim3(kMWG),
+                           lds, st, static_cast<const uint8_t *>(w), xq, xs, dst, (int)m, (int)n,
                            (int)k, mt, nt, (int)split_k, ts);
-    else if (aligned)
-        hipLaunchKernelGGL((mmq_kernel<true, HOUT>), dim3(grid_x, split_k), dim3(kMWG), lds, st,
-                           static_cast<const uint8_t *>(w), xq, xs, dst, (int)m, (int)n, (int)k,
-                           mt, nt, (int)split_k, ts);
     else
-        hipLaunchKernelGGL((mmq_kernel<false, HOUT>), dim3(grid_x, split_k), dim3(kMWG), lds, st,
-                           static_cast<const uint8_t *>(w), xq, xs, dst, (int)m, (int)n, (int)k,
-                           mt, nt, (int)split_k, ts);
+        hipLaunchKernelGGL((mmq_kernel<HOUT>), dim3(grid_x, split_k), dim3(kMWG), lds, st,
+                           static_cast<const uint8_t *>(w), xq, xs, dst, (int)m, (int)n, (int)k, mt,
+                           nt, (int)split_k, ts);
     SGQ_HIP(hipGetLastError());
     if (ts.st) {
         const int tail_tiles = kXcds * (tiles / kXcds - ts.fx);
         hipLaunchKernelGGL(mmq_tail_reduce_kernel, dim3(tail_tiles * 16), dim3(256), 0, st, ts,
-                           static_cast<float *>(y), (int)n, mt, nt);
+                           static_cast<float *>(y), (int)m, (int)n, mt, nt);
         SGQ_HIP(hipGetLastError());
     }
     if (split_k > 1) {

@@ -56,6 +56,33 @@ def test_mmq_small_full_check(ctx, oracle, m, k, n):
     assert rel_err(got, want) <= 2e-6
 
 
+@pytest.mark.parametrize("m,k,n,split", [
+    (1, 64, 1, 1), (33, 64, 127, 1), (127, 192, 129, 1), (129, 448, 256, 1), (256, 1216, 128, 1),
+    (128, 320, 131, 1), (65, 1088, 132, 4), (300, 2112, 260, 8)])
+def test_mmq_tile_and_k_edges(ctx, oracle, m, k, n, split):
+    """Rows and columns around the tile edges with a K that ends in two
+    blocks (k % 128 == 64, one stage at K = 64), whole and split over K:
+    every element against the oracle, the operands at the very end of their
+    buffers and the output's surroundings untouched."""
+    print(f"mmq edges m={m} k={k} n={n} split={split}", flush=True)
+    rng = oracle.Rng(0xED6E + m + k + n)
+    w = rng.random_q4_0(n * k // 32)
+    x = oracle.through_f16(rng.f32_vec(m * k))
+    xq_t, xs_t = _quant_on_gpu(ctx, dev(x), m, k)
+    pad = 256
+    buf = torch.full((m * n + 2 * pad,), float("nan"), dtype=torch.float32, device="cuda")
+    part = empty(split * m * n, torch.float32) if split > 1 else None
+    ctx.gemm_q4_0_q8(dev(w), xq_t, xs_t, buf[pad:pad + m * n], m, n, k, split, part)
+    torch.cuda.synchronize()
+    got = host(buf)
+    assert np.isnan(got[:pad]).all() and np.isnan(got[pad + m * n:]).all()
+    got = got[pad:pad + m * n].reshape(m, n)
+    want = oracle.mmq_q4_0_q8(w, x, m, k, n)
+    rms = float(np.sqrt(np.mean(want.astype(np.float64) ** 2)))
+    assert_close(got, want, 1e-3, 1e-4 * rms, f"mmq {m}x{k}x{n}")
+    assert rel_err(got, want) <= 2e-6
+
+
 def test_mmq_integer_tile_is_exact(ctx, oracle):
     """coop_i8_smoke (crates/sg-gpu/tests/coop_i8_smoke.rs) inputs
     a[i][k] = (i+k)%7-3, b[k][j] = (k*j)%11-5 on a 16×16×16 tile, padded to
