@@ -480,9 +480,186 @@ __global__ __launch_bounds__(256) void mmq_tail_reduce_kernel(TailSplit ts, floa
     *reinterpret_cast<float4 *>(y + (size_t)(tm * BM + row) * n + tn * BN + 4 * c4) = a;
 }
 
+// Few rows (m <= 32·TM): one workgroup per 32 columns computes all rows, its W
+// waves each a contiguous range of K, so that even a narrow matrix has waves
+// on every CU and its weights stream once; the waves' sums meet in LDS, in
+// wave order.  A step is 4 blocks: each wave loads its 32 columns' 72 bytes
+// and its rows' 128 bytes with consecutive lanes on consecutive addresses
+// (a lane per row instead touched 32 cache lines per load, and that bounded
+// the kernel), one step ahead in registers, and turns them into MFMA operands
+// through an LDS tile of its own (no barriers in the loop).
+template <int TM, int W, bool HOUT>
+__global__ __launch_bounds__(W * 64, 2) void mmq_skinny_kernel(
+    const uint8_t *__restrict__ W_, const int8_t *__restrict__ xq, const uint16_t *__restrict__ xs,
+    void *__restrict__ out_, int m, int n, int k) {
+    constexpr int kABytes = TM * 32 * 128, kBWords = 32 * 18;
+    constexpr int kWaveBytes = kABytes + kBWords * 4;
+    constexpr int kRedBytes = TM * 16 * 64 * 4;
+    __shared__ __align__(16) uint8_t lds[W * (kWaveBytes > kRedBytes ? kWaveBytes : kRedBytes)];
+    const int nb = k / 32, ns = (nb + KB - 1) / KB;  // nb is even
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 31, h = lane >> 5;
+    const int n0 = blockIdx.x * 32;
+    const int s0 = (int)((long)ns * wave / W), s1 = (int)((long)ns * (wave + 1) / W);
+    uint8_t *la = lds + wave * kWaveBytes;
+    uint32_t *lb = reinterpret_cast<uint32_t *>(la + kABytes);
+
+    // load offsets from the step's first block; a K of 64 (one step with one
+    // live pair) reads the live bytes again in place of the dead ones
+    const int live_blocks = min(nb, KB);
+    uint32_t ob[9], oa[4 * TM], od[TM];
+#pragma unroll
+    for (int i = 0; i < 9; i++) {
+        const int d = i * 64 + lane, col = d / 18, e = min(d % 18, live_blocks * 9 / 2 - 1);
+        ob[i] = (uint32_t)min(col, n - 1 - n0) * (uint32_t)nb * 18 + 4 * e;
+    }
+#pragma unroll
+    for (int i = 0; i < 4 * TM; i++)
+        oa[i] = (uint32_t)min(8 * i + (lane >> 3), m - 1) * (uint32_t)k +
+                16 * min(lane & 7, 2 * live_blocks - 1);
+#pragma unroll
+    for (int i = 0; i < TM; i++) od[i] = (uint32_t)min(32 * i + r, m - 1) * (uint32_t)nb * 2;
+    const uint32_t od2 = nb < KB ? 0 : 4;
+    // LDS: activation chunk c (16 bytes) of row x at slot c ^ (x % 8), so the
+    // operand reads of 8 lanes fall on distinct banks; weights as loaded
+    uint8_t *wa = la + ((lane & ~7) + ((lane & 7) ^ (lane >> 3))) * 16;
+    const uint8_t *ra = la + r * 128;
+    const uint32_t rx = (uint32_t)(h ^ (r & 7)) * 16;
+    const uint32_t *rb = lb + r * 18;
+
+    v4i ga[4 * TM];
+    uint32_t gb[9];
+    uint2 gs[TM];
+    // a K end with two blocks: the last step starts two blocks early and the
+    // pair it repeats has zero scales (K of 64: the second pair)
+    const bool short_end = nb % KB != 0;
+    const int dead = nb < KB ? 1 : 0;
+    auto load = [&](int st) {
+        const int b0 = short_end && !dead && st + 1 == ns ? nb - KB : st * KB;
+        gptr a = (gptr)xq + (size_t)b0 * 32, d = (gptr)xs + (size_t)b0 * 2;
+        gptr w = (gptr)W_ + ((size_t)n0 * nb + b0) * 18;
+        asm volatile("" : "+s"(a), "+s"(w), "+s"(d));
+#pragma unroll
+        for (int i = 0; i < 9; i++) {
+            uint32_t o = ob[i];
+            asm volatile("" : "+v"(o));
+            gb[i] = *(const __attribute__((address_space(1))) uint32_t *)(w + o);
+        }
+#pragma unroll
+        for (int i = 0; i < 4 * TM; i++) {
+            uint32_t o = oa[i];
+            asm volatile("" : "+v"(o));
+            ga[i] = *(const __attribute__((address_space(1))) v4i *)(a + o);
+        }
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            uint32_t o = od[i];
+            asm volatile("" : "+v"(o));
+            gs[i] = make_uint2(*(const __attribute__((address_space(1))) u32a2 *)(d + o),
+                               *(const __attribute__((address_space(1))) u32a2 *)(d + o + od2));
+        }
+    };
+    f32x16 acc[TM];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int q = 0; q < 16; q++) acc[i][q] = 0.f;
+    const uint32_t sh = h ? 0 : 4;           // this half's nibbles to the bytes' high halves
+    const uint32_t live = h ? 0u : 0xffffu;  // the scale MFMA's one live K term (h = 0)
+    if (s0 < s1) load(s0);
+#pragma unroll 1
+    for (int st = s0; st < s1; st++) {
+        const bool cut = short_end && st + 1 == ns;
+#pragma unroll
+        for (int i = 0; i < 4 * TM; i++) *reinterpret_cast<v4i *>(wa + i * 1024) = ga[i];
+#pragma unroll
+        for (int i = 0; i < 9; i++) lb[i * 64 + lane] = gb[i];
+        uint32_t sa[TM][2];
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            sa[i][0] = cut && !dead ? 0u : gs[i].x;
+            sa[i][1] = cut && dead ? 0u : gs[i].y;
+        }
+        if (st + 1 < s1) load(st + 1);
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            uint32_t w[9];
+#pragma unroll
+            for (int e = 0; e < 9; e++) w[e] = rb[9 * p + e];
+            const uint32_t lw = cut && p == dead ? 0u : live;
+#pragma unroll
+            for (int blk = 0; blk < 2; blk++) {
+                v4i bf;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const uint32_t q = blk ? w[5 + e] : __builtin_amdgcn_alignbyte(w[e + 1], w[e], 2);
+                    bf[e] = (int)(((q << sh) & 0xF0F0F0F0u) ^ 0x80808080u);
+                }
+                const h4 bs = __builtin_bit_cast(h4, v2i{(int)((blk ? w[4] >> 16 : w[0]) & lw), 0});
+#pragma unroll
+                for (int i = 0; i < TM; i++) {
+                    const v4i af = *reinterpret_cast<const v4i *>(
+                        ra + i * 4096 + (rx ^ (32u * (2 * p + blk))));
+                    const h4 as = __builtin_bit_cast(
+                        h4, v2i{(int)((blk ? sa[i][p] >> 16 : sa[i][p]) & live), 0});
+                    const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, bf, v16i{}, 0, 0, 0);
+                    const f32x16 sc = __builtin_amdgcn_mfma_f32_32x32x8f16(as, bs, f32x16{}, 0, 0, 0);
+#pragma unroll
+                    for (int q = 0; q < 16; q++)
+                        acc[i][q] = __builtin_fmaf((float)d[q], sc[q], acc[i][q]);
+                }
+            }
+        }
+    }
+    __syncthreads();  // every wave is done with its tile
+    float(*red)[TM * 16 * 64] = reinterpret_cast<float(*)[TM * 16 * 64]>(lds);
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int q = 0; q < 16; q++) red[wave][(i * 16 + q) * 64 + lane] = acc[i][q];
+    __syncthreads();
+    // element e of the workgroup's rows: (row tile, q, lane)
+    for (int e = threadIdx.x; e < TM * 1024; e += W * 64) {
+        float v = red[0][e];
+#pragma unroll
+        for (int z = 1; z < W; z++) v += red[z][e];
+        v *= kUnscale;
+        const int l = e & 63, q = (e >> 6) & 15, i = e >> 10;
+        const int row = 32 * i + 8 * (q / 4) + 4 * (l >> 5) + (q % 4), col = n0 + (l & 31);
+        if (row < m && col < n) {
+            if (HOUT)
+                static_cast<uint16_t *>(out_)[(size_t)row * n + col] = f32_to_f16_bits(v);
+            else
+                static_cast<float *>(out_)[(size_t)row * n + col] = v;
+        }
+    }
+}
+
 }  // namespace
 
 namespace {
+template <int TM, int W, bool HOUT>
+void skinny_launch(hipStream_t st, const void *w, const int8_t *xq, const uint16_t *xs, void *y,
+                   uint32_t m, uint32_t n, uint32_t k) {
+    hipLaunchKernelGGL((mmq_skinny_kernel<TM, W, HOUT>), dim3((n + 31) / 32), dim3(W * 64), 0, st,
+                       static_cast<const uint8_t *>(w), xq, xs, y, (int)m, (int)n, (int)k);
+}
+
+// The few-rows kernel against the tiles, whose launch of one round costs the
+// same for 1 row as for 128 (81 us at K = 5376; 310 at K = 21504, or 69 split
+// over K 8 ways).  us at N = 21504, K = 5376 / N = 5376, K = 21504, tiles at
+// split 1 81 / 310: M = 1 21 / 26, 37 35 / 43, 64 38 / 48, 100 77 / 87.  Its
+// time grows with n by 1.0 / 1.8 / 3.6 us per 1000 columns (M <= 32 / 64 /
+// 128, K = 5376) where the tiles' stays until their round of 65536 columns is
+// full, hence the limits on n; above 64 rows a caller's split over K is the
+// faster of the two.
+bool skinny(uint32_t m, uint32_t n, uint32_t split_k) {
+    if (m <= 32) return true;
+    if (m <= 64) return n <= 43008;
+    return m <= 128 && n <= 21504 && split_k == 1;
+}
+
 template <bool HOUT>
 int gemm_t(hipStream_t st, const void *w, const int8_t *xq, const uint16_t *xs, void *y,
            uint32_t m, uint32_t n, uint32_t k, uint32_t split_k, float *partials) {
@@ -496,6 +673,27 @@ int gemm_t(hipStream_t st, const void *w, const int8_t *xq, const uint16_t *xs, 
     SGQ_CHECK(((uintptr_t)w & 3) == 0, "gemm_q4_0_q8: weights must be 4-byte aligned");
     SGQ_CHECK((uint64_t)m * n < (1ull << 31) * 4, "gemm_q4_0_q8: output too large");
     SGQ_CHECK(split_k == 1 || (m * (uint64_t)n) % 4 == 0, "gemm_q4_0_q8: m*n must be a multiple of 4 for split-K");
+    if (k < kWideK && skinny(m, n, split_k)) {
+        // W: 8 waves cut a column tile's K finer (N = 5376, K = 21504, M = 37:
+        // 43 against 69 us); with two tiles or more per CU, 4 leave smaller
+        // workgroups to even out over the CUs (N = 21504, M = 37: 35 against 45)
+        const bool w4 = n >= 16384;
+        const int tm = (int)(m + 31) / 32;
+#define SGQ_SKINNY(TM)                                                          \
+    (w4 ? skinny_launch<TM, 4, HOUT>(st, w, xq, xs, y, m, n, k)                  \
+        : skinny_launch<TM, 8, HOUT>(st, w, xq, xs, y, m, n, k))
+        if (tm == 1)
+            SGQ_SKINNY(1);
+        else if (tm == 2)
+            SGQ_SKINNY(2);
+        else if (tm == 3)
+            SGQ_SKINNY(3);
+        else
+            SGQ_SKINNY(4);
+#undef SGQ_SKINNY
+        SGQ_HIP(hipGetLastError());
+        return SGQ_OK;
+    }
     static bool attr = false;
     const size_t lds = 2 * sizeof(Stage);
     if (!attr) {

@@ -58,12 +58,16 @@ def test_mmq_small_full_check(ctx, oracle, m, k, n):
 
 @pytest.mark.parametrize("m,k,n,split", [
     (1, 64, 1, 1), (33, 64, 127, 1), (127, 192, 129, 1), (129, 448, 256, 1), (256, 1216, 128, 1),
-    (128, 320, 131, 1), (65, 1088, 132, 4), (300, 2112, 260, 8)])
+    (128, 320, 131, 1), (65, 1088, 132, 4), (300, 2112, 260, 8),
+    (16, 128, 31, 1), (31, 2112, 96, 8), (32, 64, 33, 1), (64, 1088, 65, 2), (96, 192, 64, 1),
+    (97, 576, 37, 1), (2, 192, 16390, 1), (40, 128, 16385, 1)])
 def test_mmq_tile_and_k_edges(ctx, oracle, m, k, n, split):
     """Rows and columns around the tile edges with a K that ends in two
     blocks (k % 128 == 64, one stage at K = 64), whole and split over K:
     every element against the oracle, the operands at the very end of their
-    buffers and the output's surroundings untouched."""
+    buffers and the output's surroundings untouched.  Up to 64 rows (128
+    unsplit) the few-rows kernel answers: its row tiles' edges, K ranges
+    shorter than its waves, and both workgroup sizes."""
     print(f"mmq edges m={m} k={k} n={n} split={split}", flush=True)
     rng = oracle.Rng(0xED6E + m + k + n)
     w = rng.random_q4_0(n * k // 32)
