@@ -136,3 +136,71 @@ def test_elementwise_bit_deterministic(ctx, oracle):
     ctx.rmsnorm(x, w, b, rows, row_len)
     torch.cuda.synchronize()
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("row_len,rows", [
+    (4, 9), (124, 17), (128, 8), (132, 5), (256, 3), (260, 7), (512, 4), (516, 2), (5376, 512),
+    (5376, 513), (6144, 513), (6148, 513), (8192, 2), (8196, 2), (130, 3)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_rmsnorm_forms_match_oracle(ctx, oracle, row_len, rows, shift):
+    """The three norm kernels at the row lengths and row counts where the
+    choice changes, and from a pointer off the 16-byte alignment (shift 1: the
+    scalar form), nothing written around the rows."""
+    print(f"rmsnorm {rows} x {row_len} shift {shift}", flush=True)
+    rng = oracle.Rng(0xE7 + row_len + rows)
+    n = rows * row_len
+    x, w = rng.f32_vec(n) * np.float32(3.0), rng.f32_vec(row_len)
+    tx = torch.empty(n + 1, dtype=torch.float32, device="cuda")[shift:shift + n]
+    tx.copy_(torch.from_numpy(x))
+    buf = torch.full((n + 64,), float("nan"), dtype=torch.float32, device="cuda")
+    y = buf[32 + shift:32 + shift + n]
+    ctx.rmsnorm(tx, dev(w), y, rows, row_len)
+    torch.cuda.synchronize()
+    _close(host(y), oracle.rmsnorm(x, w, row_len, 1e-6, False), f"rmsnorm {row_len}x{rows}")
+    got = host(buf)
+    assert np.isnan(got[:32 + shift]).all() and np.isnan(got[32 + shift + n:]).all()
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 8, 1023, 1024, 1029, 4099])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_binary_streams_edges(ctx, oracle, n, shift):
+    """GeGLU and add_scaled at the ends of a 16-byte vector and of a workgroup,
+    aligned and not; GeGLU over large arguments of both signs and zero."""
+    print(f"binary n={n} shift={shift}", flush=True)
+    rng = oracle.Rng(0xE8 + n)
+    g, u = rng.f32_vec(n) * np.float32(8.0), rng.f32_vec(n)
+    g[::5] *= np.float32(100.0)
+    g[n // 2] = 0.0
+
+    def place(a):
+        t = torch.empty(n + 1, dtype=torch.float32, device="cuda")[shift:shift + n]
+        t.copy_(torch.from_numpy(a))
+        return t
+
+    for name in ("geglu", "add"):
+        buf = torch.full((n + 64,), float("nan"), dtype=torch.float32, device="cuda")
+        y = buf[32 + shift:32 + shift + n]
+        if name == "geglu":
+            ctx.geglu(place(g), place(u), y)
+            want = oracle.geglu(g, u)
+        else:
+            ctx.add_scaled(place(g), place(u), y, 0.75)
+            want = oracle.add_scaled(g, u, 0.75)
+        torch.cuda.synchronize()
+        _close(host(y), want, name)
+        got = host(buf)
+        assert np.isnan(got[:32 + shift]).all() and np.isnan(got[32 + shift + n:]).all()
+
+
+@pytest.mark.parametrize("head_dim,rot,n_heads", [(24, 8, 3), (24, 12, 3), (20, 8, 2), (512, 128, 4)])
+def test_rope_vector_and_scalar_forms(ctx, oracle, head_dim, rot, n_heads):
+    """Four pairs per thread where head and rotation are whole quads of pairs,
+    one per thread elsewhere: the same values."""
+    n_tok = 3
+    rng = oracle.Rng(0xE9 + head_dim + rot)
+    x = rng.f32_vec(n_tok * n_heads * head_dim)
+    cs = rng.f32_vec(n_tok * rot).reshape(n_tok, rot // 2, 2)
+    tx = dev(x)
+    ctx.rope(tx, dev(cs), n_tok, n_heads, head_dim, rot)
+    torch.cuda.synchronize()
+    _close(host(tx), oracle.rope(x, head_dim, rot, n_heads, cs), "rope")
