@@ -722,7 +722,8 @@ __global__ __launch_bounds__(256 * HPW + 256) void attn_prefill_ws_kernel(
 //           the integer dot exact on the f16 MFMA
 //           (attn_prefill_global_flash_sp_ipv.wgsl:134-210)
 // Except for kPfQ8, q enters the MFMA as its exact f16 values and the
-// scores are scaled afterwards.
+// scores are scaled afterwards.  attn_prefill_px_kernel (below) serves kPfQ8H,
+// kPfF16 and all but the shortest kPfQ8.
 enum PfFmt { kPfQ8 = 0, kPfQ8H = 1, kPfF16 = 2, kPfIQ = 3, kPfIPV = 4 };
 
 template <int HD, int FMT>
@@ -730,11 +731,11 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
     const void *__restrict__ qv, const uint16_t *__restrict__ q_scales, KvSource src,
     void *__restrict__ outv, int n_tok, int q0_host, const uint32_t *__restrict__ step, int n_q,
     int n_kv, int window, float scale, int qtiles) {
+    static_assert(FMT == kPfQ8 || FMT == kPfIQ || FMT == kPfIPV, "the others: attn_prefill_px_kernel");
     constexpr bool VKB = FMT == kPfIPV;  // int8 V, key-blocked scales, int8 P
-    constexpr bool QF32 = FMT == kPfQ8, QI8 = FMT == kPfIQ || VKB;
-    constexpr bool KQ8 = FMT == kPfQ8 || FMT == kPfQ8H;  // dequantized into LDS
-    constexpr bool KF16 = FMT == kPfF16, KRAW = FMT == kPfIQ || VKB;
-    constexpr bool VF16 = FMT == kPfF16 || FMT == kPfIQ;
+    constexpr bool QF32 = FMT == kPfQ8, KQ8 = QF32;  // K dequantized into LDS
+    constexpr bool KRAW = !QF32;                     // int8 q and K, scaled after the dots
+    constexpr bool VF16 = FMT == kPfIQ;
     constexpr bool O16 = FMT != kPfQ8;
     constexpr int D = HD / 128;        // waves per query tile
     constexpr int QTW = 8 / D;         // query tiles per workgroup
@@ -788,7 +789,7 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
 #pragma unroll
                 for (int e = 0; e < 8; e++) qb[c][e] = (_Float16)(q_valid ? v[e] * qscale : 0.f);
             }
-        } else if constexpr (QI8) {
+        } else {
             const int8_t *qr = static_cast<const int8_t *>(qv) + qoff;
 #pragma unroll
             for (int c = 0; c < 8; c++) {
@@ -802,13 +803,6 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
 #pragma unroll
             for (int b = 0; b < 4; b++)
                 qsb[b] = q_valid ? (float)__builtin_bit_cast(_Float16, qs[b]) * qscale : 0.f;
-        } else {
-            const uint16_t *qr = static_cast<const uint16_t *>(qv) + qoff;
-#pragma unroll
-            for (int c = 0; c < 8; c++) {
-                const h8 t = __builtin_bit_cast(h8, *reinterpret_cast<const uint4 *>(qr + 16 * c));
-                qb[c] = q_valid ? t : h8{};
-            }
         }
     }
 
@@ -829,7 +823,7 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
     // dims CW·chunk .. +CW-1
     const int pair = tid % NP, chunk = tid / NP;
     const int dim0 = CW * chunk, blk = dim0 >> 5;
-    constexpr int EK = KF16 ? 2 : 1, EV = VF16 ? 2 : 1;  // bytes per K / V element
+    constexpr int EV = VF16 ? 2 : 1;  // bytes per V element (K: 1)
     const char *const kq_c = sgpr_ptr(reinterpret_cast<const char *>(src.kq));
     const char *const vq_c = sgpr_ptr(reinterpret_cast<const char *>(src.vq));
     const uint16_t *const ks_c = sgpr_ptr(src.ks), *const vs_c = sgpr_ptr(src.vs);
@@ -839,7 +833,7 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
     const uint16_t *const ks_f = has_chunk ? sgpr_ptr(src.cks) : ks_c;
     const uint16_t *const vs_f = has_chunk ? sgpr_ptr(src.cvs) : vs_c;
     const int ring = src.ring;
-    typedef int kraw_t __attribute__((ext_vector_type(CW * EK / 4)));
+    typedef int kraw_t __attribute__((ext_vector_type(CW / 4)));
     typedef int vraw_t __attribute__((ext_vector_type(CW * EV / 4)));
     kraw_t rk[2];
     vraw_t rv[2];
@@ -852,9 +846,9 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
             const bool fresh = has_chunk && key >= q0;
             const int slot = fresh ? key - q0 : ring ? key % ring : key;
             const size_t row = (size_t)slot * n_kv + kvh;
-            rk[e] = gload(reinterpret_cast<const kraw_t *>((fresh ? kq_f : kq_c) + (row * HD + dim0) * EK));
+            rk[e] = gload(reinterpret_cast<const kraw_t *>((fresh ? kq_f : kq_c) + row * HD + dim0));
             rv[e] = gload(reinterpret_cast<const vraw_t *>((fresh ? vq_f : vq_c) + (row * HD + dim0) * EV));
-            if constexpr (!KF16) rsk[e] = gload((fresh ? ks_f : ks_c) + row * NB + blk);
+            rsk[e] = gload((fresh ? ks_f : ks_c) + row * NB + blk);
             if constexpr (!VF16 && !VKB) rsv[e] = gload((fresh ? vs_f : vs_c) + row * NB + blk);
         }
         if constexpr (VKB)
@@ -873,30 +867,22 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
             const bool live = kl + kk <= k_hi;
             h8 kt[CW / 8];
             _Float16 vv[CW];
-            if constexpr (KF16) {
+            const _Float16 sk = KQ8 && live ? __builtin_bit_cast(_Float16, rsk[e]) : (_Float16)1.f;
+            const h2 dk = {sk, sk};
 #pragma unroll
-                for (int h = 0; h < CW / 8; h++) {
-                    const int4 w = {rk[e][4 * h], rk[e][4 * h + 1], rk[e][4 * h + 2], rk[e][4 * h + 3]};
-                    kt[h] = live ? __builtin_bit_cast(h8, w) : h8{};
-                }
-            } else {
-                const _Float16 sk = KQ8 && live ? __builtin_bit_cast(_Float16, rsk[e]) : (_Float16)1.f;
-                const h2 dk = {sk, sk};
-#pragma unroll
-                for (int w = 0; w < CW / 4; w++) {
-                    h2 k01 = i8_pair_f16((uint32_t)rk[e][w], 0x04010400u);
-                    h2 k23 = i8_pair_f16((uint32_t)rk[e][w], 0x04030402u);
-                    if constexpr (KQ8) k01 *= dk, k23 *= dk;
-                    kt[w / 2][4 * (w & 1)] = k01[0], kt[w / 2][4 * (w & 1) + 1] = k01[1];
-                    kt[w / 2][4 * (w & 1) + 2] = k23[0], kt[w / 2][4 * (w & 1) + 3] = k23[1];
-                }
-                if (!live)
-#pragma unroll
-                    for (int h = 0; h < CW / 8; h++) kt[h] = h8{};
-                if constexpr (KRAW)
-                    if (dim0 % 32 == 0)
-                        ksc_s[blk][kk] = live ? (float)__builtin_bit_cast(_Float16, rsk[e]) : 0.f;
+            for (int w = 0; w < CW / 4; w++) {
+                h2 k01 = i8_pair_f16((uint32_t)rk[e][w], 0x04010400u);
+                h2 k23 = i8_pair_f16((uint32_t)rk[e][w], 0x04030402u);
+                if constexpr (KQ8) k01 *= dk, k23 *= dk;
+                kt[w / 2][4 * (w & 1)] = k01[0], kt[w / 2][4 * (w & 1) + 1] = k01[1];
+                kt[w / 2][4 * (w & 1) + 2] = k23[0], kt[w / 2][4 * (w & 1) + 3] = k23[1];
             }
+            if (!live)
+#pragma unroll
+                for (int h = 0; h < CW / 8; h++) kt[h] = h8{};
+            if constexpr (KRAW)
+                if (dim0 % 32 == 0)
+                    ksc_s[blk][kk] = live ? (float)__builtin_bit_cast(_Float16, rsk[e]) : 0.f;
             if constexpr (VF16) {
 #pragma unroll
                 for (int w = 0; w < CW / 2; w++) {
@@ -996,9 +982,6 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
             }
             s[4 * j] = t.x, s[4 * j + 1] = t.y, s[4 * j + 2] = t.z, s[4 * j + 3] = t.w;
         }
-        if constexpr (!QF32 && !KRAW)
-#pragma unroll
-            for (int i = 0; i < 16; i++) s[i] *= qscale;
         const uint32_t *vt = vt_s[buf];
         {
             const int kb = kl;
@@ -1113,6 +1096,371 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
         }
 }
 
+// The value of the lane 32 (16) away beside one's own, without the LDS trip of
+// a shuffle: {lanes 0-31 / even rows of 16, lanes 32-63 / odd rows} in both.
+__device__ __forceinline__ float max_x32(float v) {
+    const uint32_t b = __builtin_bit_cast(uint32_t, v);
+    const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    return fmaxf(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
+}
+__device__ __forceinline__ float max_x16(float v) {
+    const uint32_t b = __builtin_bit_cast(uint32_t, v);
+    const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    return fmaxf(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
+}
+
+// Prefill attention at head_dim 256 / 512 without repeated scores: one query
+// head per workgroup of 8 waves, D = head_dim/128 waves per tile of 32 queries.
+// A tile's scores are cut between its D waves by (key, query), over all dims,
+// so that no score is computed, masked or exponentiated twice:
+//   head_dim 256 (KT = 64): wave ds takes 32 keys × 32 queries
+//                           (v_mfma_f32_32x32x16_f16);
+//   head_dim 512 (KT = 32): wave ds takes 16 keys × 16 queries
+//                           (v_mfma_f32_16x16x32_f16).
+// Each wave writes its P as f16 and the reference max it used to LDS; after
+// the barrier every wave reads the tile's whole P as the B operand of
+// Oᵀ = Vᵀ·Pᵀ for its own 128 dims.  A reference is the query's maximum over the
+// first tile (exchanged there, one more barrier) and moves rarely (lazily, by
+// more than 2^8) and by whole powers of two, so that bringing the parts of P to
+// their common one is exact.  The denominator sums P as rounded to f16, as the
+// numerator does.
+// Per tile: scores, P out → barrier → PV(t), K(t+1) and V(t+1) staged from
+// registers (V double-buffered), quants of t+2 issued → barrier.
+// It replaces attn_prefill_wide_kernel, whose D waves each compute partial
+// scores over 128 dims, exchange them as f32 and repeat the softmax, for the
+// f16 and Q8_0 formats (us, before -> after; kv heads 16 / 4): head_dim 256,
+// Q8_0, 1024 window, 4096 queries 401 -> 306, 1111 queries from 2003 196 ->
+// 155; f16 ring, 512 queries from 1777 84 -> 72; head_dim 512, Q8_0, causal,
+// 2000 queries 406 -> 365, 20 queries from 3000 259 -> 195; f16, 1024 queries
+// from 1000 290 -> 257.  What bounds it: waits between dependent LDS reads and
+// MFMAs (two waves per SIMD), then the dequant's VALU.  Two forms with fewer
+// waves per score measured slower: 256 dims per wave (spills; f16 ring of 2048
+// queries 199 against 145), all dims in one wave per SIMD with Oᵀ in
+// accumulation registers (1029 for the 1111 queries).  Int8 q stays with the
+// wide kernel: here its block scales spill (322 -> 1020 for 1024 queries from
+// 1024).
+template <int HD, int FMT>
+__global__ __launch_bounds__(512, 2) void attn_prefill_px_kernel(
+    const void *__restrict__ qv, const uint16_t *__restrict__ q_scales, KvSource src,
+    void *__restrict__ outv, int n_tok, int q0_host, const uint32_t *__restrict__ step, int n_q,
+    int n_kv, int window, float scale, int qtiles) {
+    constexpr bool QF32 = FMT == kPfQ8, F16 = FMT == kPfF16, O16 = FMT != kPfQ8;
+    static_assert(QF32 || F16 || FMT == kPfQ8H, "Q8_0 or f16 pages, fp32 or f16 q");
+    constexpr bool S32 = HD == 256;           // scores as a 32×32 tile (else 16×16)
+    constexpr int D = HD / 128;               // waves per query tile
+    constexpr int QW = 32 * (8 / D);          // queries per workgroup
+    constexpr int KT = S32 ? 64 : 32;         // keys per tile
+    constexpr int NB = HD / 32, NP = KT / 2, CW = 16;
+    static_assert(NP * (HD / CW) == 512, "one staging item per thread");
+    constexpr int KRowB = (HD + 8) * 2;       // bytes per K row (f16) in LDS
+    constexpr int VS = NP + 4;                // Vᵀ row, dwords (16-byte reads, 4 banks apart)
+    constexpr int VPad = S32 ? 0 : 16;        // dwords per 16 rows: the staging writes of a wave
+    constexpr int VBuf = HD * VS + (HD / 16) * VPad;
+    constexpr int PRow = KT + 8;              // P row (halves): [query][key]
+    constexpr int kKBytes = KT * KRowB, kVBytes = 2 * VBuf * 4, kPBytes = QW * PRow * 2;
+    constexpr int kMBytes = 4 * QW * 4;       // [key part][query]: reference maxima, first maxima
+    __shared__ __align__(16) uint8_t lds[kKBytes + kVBytes + kPBytes + kMBytes];
+    uint8_t *const k_lds = lds;
+    uint32_t *const v_lds = reinterpret_cast<uint32_t *>(lds + kKBytes);
+    uint16_t *const p_lds = reinterpret_cast<uint16_t *>(lds + kKBytes + kVBytes);
+    float *const m_lds = reinterpret_cast<float *>(lds + kKBytes + kVBytes + kPBytes);
+    auto vt_at = [](int row, int col) { return row * VS + (row >> 4) * VPad + col; };
+
+    int bx = (int)blockIdx.x, by = (int)blockIdx.y;
+    if (gridDim.y % 8 == 0) {  // XCD-aware order, as in attn_prefill_kernel
+        const int L = bx + by * qtiles, per = (int)gridDim.y / 8, idx = L >> 3;
+        by = (L & 7) * per + idx % per;
+        bx = idx / per;
+    }
+    const int q0 = QF32 ? q0_host : (int)step[3];
+    const int tile = qtiles - 1 - bx;  // heaviest (latest) query tile first
+    const int qh = by, kvh = qh / (n_q / n_kv);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int qt = wave / D, ds = wave % D;
+    const int l32 = lane & 31, hh = lane >> 5;
+    // this wave's scores: key part kp (of 2), and this lane's score query sq
+    // (of the tile's 32); A / B operand row within the part and K quarter
+    const int kp = S32 ? ds : ds >> 1;
+    const int sq = S32 ? l32 : 16 * (ds & 1) + (lane & 15);
+    const int orow = S32 ? l32 : lane & 15, okq = S32 ? hh : lane >> 4;
+    const int tq0 = tile * QW + qt * 32;     // the query tile's first query
+    const int my_s = tq0 + sq;
+    const bool s_valid = my_s < n_tok;
+    const int sp = q0 + my_s;                // the score query's position
+
+    const float qscale = scale * 1.44269504088896341f;
+    constexpr int NC = S32 ? HD / 16 : HD / 32;  // MFMA steps over the dims
+    h8 qb[NC];
+    {
+        const size_t row = (size_t)(s_valid ? my_s : 0) * n_q + qh;
+        if constexpr (QF32) {
+            const float *qr = static_cast<const float *>(qv) + row * HD + 8 * okq;
+#pragma unroll
+            for (int c = 0; c < NC; c++) {
+                const float4 x = *reinterpret_cast<const float4 *>(qr + (HD / NC) * c);
+                const float4 y = *reinterpret_cast<const float4 *>(qr + (HD / NC) * c + 4);
+                const float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+#pragma unroll
+                for (int e = 0; e < 8; e++) qb[c][e] = (_Float16)(s_valid ? v[e] * qscale : 0.f);
+            }
+        } else {
+            const uint16_t *qr = static_cast<const uint16_t *>(qv) + row * HD + 8 * okq;
+#pragma unroll
+            for (int c = 0; c < NC; c++) {
+                const h8 t = __builtin_bit_cast(h8, *reinterpret_cast<const uint4 *>(qr + (HD / NC) * c));
+                qb[c] = s_valid ? t : h8{};
+            }
+        }
+    }
+    f32x16 o[4];
+#pragma unroll
+    for (int d = 0; d < 4; d++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) o[d][i] = 0.f;
+    // reference maxima of the score query and of the output query (l32), and
+    // the output query's sum over this half's keys
+    float m_s = kNegBig, m_o = kNegBig, l_run = 0.f;
+
+    const int qpos_lo = q0 + tile * QW;
+    const int k_hi = q0 + min((tile + 1) * QW, n_tok) - 1;
+    const int k_lo = window > 0 ? max(0, qpos_lo + 1 - window) : 0;
+    const int tq_lo = q0 + tq0, tq_hi = min(tq_lo + 31, k_hi);  // the tile's live positions
+
+    // staging item of this thread: keys 2·pair, 2·pair + 1 of the tile, dims
+    // dim0 .. +15
+    const int pair = tid % NP, dim0 = CW * (tid / NP), blk = dim0 >> 5;
+    constexpr int EK = F16 ? 2 : 1, EV = F16 ? 2 : 1;  // bytes per K / V element
+    const char *const kq_c = sgpr_ptr(reinterpret_cast<const char *>(src.kq));
+    const char *const vq_c = sgpr_ptr(reinterpret_cast<const char *>(src.vq));
+    const uint16_t *const ks_c = sgpr_ptr(src.ks), *const vs_c = sgpr_ptr(src.vs);
+    const bool has_chunk = src.ckq != nullptr;
+    const char *const kq_f = has_chunk ? sgpr_ptr(reinterpret_cast<const char *>(src.ckq)) : kq_c;
+    const char *const vq_f = has_chunk ? sgpr_ptr(reinterpret_cast<const char *>(src.cvq)) : vq_c;
+    const uint16_t *const ks_f = has_chunk ? sgpr_ptr(src.cks) : ks_c;
+    const uint16_t *const vs_f = has_chunk ? sgpr_ptr(src.cvs) : vs_c;
+    const int ring = src.ring;
+    typedef int kraw_t __attribute__((ext_vector_type(CW * EK / 4)));
+    typedef int vraw_t __attribute__((ext_vector_type(CW * EV / 4)));
+    kraw_t rk[2];
+    vraw_t rv[2];
+    uint16_t rsk[2], rsv[2];
+    auto fetch = [&](int kl) {
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const int key = min(kl + 2 * pair + e, k_hi);  // past k_hi: zeroed when staged
+            const bool fresh = has_chunk && key >= q0;
+            const int slot = fresh ? key - q0 : ring ? key % ring : key;
+            const size_t row = (size_t)slot * n_kv + kvh;
+            rk[e] = gload(reinterpret_cast<const kraw_t *>((fresh ? kq_f : kq_c) + (row * HD + dim0) * EK));
+            rv[e] = gload(reinterpret_cast<const vraw_t *>((fresh ? vq_f : vq_c) + (row * HD + dim0) * EV));
+            if constexpr (!F16) rsk[e] = gload((fresh ? ks_f : ks_c) + row * NB + blk);
+            if constexpr (!F16) rsv[e] = gload((fresh ? vs_f : vs_c) + row * NB + blk);
+        }
+    };
+    auto stage = [&](int kl, int buf) {
+        uint32_t *vt = v_lds + buf * VBuf;
+        uint32_t vpk[CW];
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const int kk = 2 * pair + e;
+            const bool live = kl + kk <= k_hi;
+            h8 kt[2];
+            if constexpr (F16) {
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const int4 w = {rk[e][4 * h], rk[e][4 * h + 1], rk[e][4 * h + 2], rk[e][4 * h + 3]};
+                    kt[h] = live ? __builtin_bit_cast(h8, w) : h8{};
+                }
+            } else {
+                const _Float16 sk = live ? __builtin_bit_cast(_Float16, rsk[e]) : (_Float16)0.f;
+                const h2 dk = {sk, sk};
+#pragma unroll
+                for (int w = 0; w < 4; w++) {
+                    const h2 k01 = i8_pair_f16((uint32_t)rk[e][w], 0x04010400u) * dk;
+                    const h2 k23 = i8_pair_f16((uint32_t)rk[e][w], 0x04030402u) * dk;
+                    kt[w / 2][4 * (w & 1)] = k01[0], kt[w / 2][4 * (w & 1) + 1] = k01[1];
+                    kt[w / 2][4 * (w & 1) + 2] = k23[0], kt[w / 2][4 * (w & 1) + 3] = k23[1];
+                }
+            }
+            *reinterpret_cast<h8 *>(k_lds + kk * KRowB + 2 * dim0) = kt[0];
+            *reinterpret_cast<h8 *>(k_lds + kk * KRowB + 2 * dim0 + 16) = kt[1];
+            _Float16 vv[CW];
+            if constexpr (F16) {
+#pragma unroll
+                for (int w = 0; w < CW / 2; w++) {
+                    const int word = rv[e][w];  // a plain value: bit_cast of a vector
+                                                // element reads element 0
+                    const h2 p = __builtin_bit_cast(h2, word);
+                    vv[2 * w] = live ? p[0] : (_Float16)0.f;
+                    vv[2 * w + 1] = live ? p[1] : (_Float16)0.f;
+                }
+            } else {
+                const _Float16 sv = live ? __builtin_bit_cast(_Float16, rsv[e]) : (_Float16)0.f;
+                const h2 dv = {sv, sv};
+#pragma unroll
+                for (int w = 0; w < CW / 4; w++) {
+                    const h2 v01 = i8_pair_f16((uint32_t)rv[e][w], 0x04010400u) * dv;
+                    const h2 v23 = i8_pair_f16((uint32_t)rv[e][w], 0x04030402u) * dv;
+                    vv[4 * w] = v01[0], vv[4 * w + 1] = v01[1], vv[4 * w + 2] = v23[0], vv[4 * w + 3] = v23[1];
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < CW; j++) {
+                const uint32_t bits = (uint32_t)__builtin_bit_cast(uint16_t, vv[j]);
+                vpk[j] = e == 0 ? bits : vpk[j] | (bits << 16);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < CW; j++) vt[vt_at(dim0 + j, pair)] = vpk[j];
+    };
+
+    constexpr int NS = S32 ? 16 : 4;  // scores per lane
+    typedef float sv_t __attribute__((ext_vector_type(NS)));
+    // key of score i within the tile
+    auto skey = [&](int i) { return S32 ? 32 * kp + 8 * (i / 4) + 4 * hh + (i % 4) : 16 * kp + 4 * okq + i; };
+    auto scores = [&]() {
+        const uint8_t *kr = k_lds + ((S32 ? 32 : 16) * kp + orow) * KRowB;
+        sv_t s0, s1;
+#pragma unroll
+        for (int i = 0; i < NS; i++) s0[i] = s1[i] = 0.f;
+#pragma unroll
+        for (int c = 0; c < NC; c += 2) {
+            const h8 a0 = *reinterpret_cast<const h8 *>(kr + 2 * ((HD / NC) * c + 8 * okq));
+            const h8 a1 = *reinterpret_cast<const h8 *>(kr + 2 * ((HD / NC) * (c + 1) + 8 * okq));
+            if constexpr (S32) {
+                s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, qb[c], s0, 0, 0, 0);
+                s1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, qb[c + 1], s1, 0, 0, 0);
+            } else {
+                s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, qb[c], s0, 0, 0, 0);
+                s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, qb[c + 1], s1, 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NS; i++) s0[i] += s1[i];
+        return s0;
+    };
+
+    fetch(k_lo);
+    stage(k_lo, 0);
+    if (k_lo + KT <= k_hi) fetch(k_lo + KT);
+    __syncthreads();
+    int buf = 0;
+#pragma unroll 1
+    for (int kl = k_lo; kl <= k_hi; kl += KT, buf ^= 1) {
+        // some query of the tile sees some key (the same in its D waves)
+        const bool live = tq_lo <= k_hi && kl <= tq_hi && (window <= 0 || kl + KT - 1 > tq_lo - window);
+        float m_part = m_s, mx = kNegBig;
+        sv_t s;
+        const bool full = kl + KT - 1 <= tq_lo && (window <= 0 || kl > tq_lo + 31 - window);
+        if (live) {
+            s = scores();
+            if constexpr (!QF32)
+#pragma unroll
+                for (int i = 0; i < NS; i++) s[i] *= qscale;
+            if (!full) {
+#pragma unroll
+                for (int i = 0; i < NS; i++) {
+                    const int key = kl + skey(i);
+                    const bool ok = s_valid && key <= sp && (window <= 0 || key > sp - window);
+                    s[i] = ok ? s[i] : kNegBig;
+                }
+            }
+            mx = s[0];
+#pragma unroll
+            for (int i = 1; i < NS; i++) mx = fmaxf(mx, s[i]);
+            if constexpr (!S32) mx = max_x16(mx);
+            mx = max_x32(mx);
+        }
+        if (kl == k_lo) {  // the first references, common to the parts: one more barrier
+            float *m0 = m_lds + 2 * QW + qt * 32 + sq;
+            if (live && (S32 ? hh == 0 : okq == 0)) m0[kp * QW] = mx;
+            __syncthreads();
+            if (live) m_part = fmaxf(m0[0], m0[QW]);
+        } else if (mx > m_s + 8.0f) {
+            m_part = m_s > kNegBig ? m_s + __builtin_ceilf(mx - m_s) : __builtin_ceilf(mx);
+        }
+        if (live) {
+            uint32_t pw[NS / 2];
+#pragma unroll
+            for (int i = 0; i < NS; i += 2) {
+                const float p0 = full || s[i] > kNegBig ? __builtin_amdgcn_exp2f(s[i] - m_part) : 0.f;
+                const float p1 = full || s[i + 1] > kNegBig ? __builtin_amdgcn_exp2f(s[i + 1] - m_part) : 0.f;
+                const h2 t = {(_Float16)p0, (_Float16)p1};
+                pw[i / 2] = __builtin_bit_cast(uint32_t, t);
+            }
+            uint16_t *pr = p_lds + (qt * 32 + sq) * PRow;
+#pragma unroll
+            for (int j = 0; j < NS / 4; j++)
+                *reinterpret_cast<uint2 *>(pr + skey(4 * j)) = make_uint2(pw[2 * j], pw[2 * j + 1]);
+            if (S32 ? hh == 0 : okq == 0) m_lds[kp * QW + qt * 32 + sq] = m_part;
+        }
+        __syncthreads();  // P and the maxima visible; K fully read
+        if (kl + KT <= k_hi) {
+            stage(kl + KT, buf ^ 1);
+            if (kl + 2 * KT <= k_hi) fetch(kl + 2 * KT);
+        }
+        if (live) {
+            const float *mq = m_lds + qt * 32;
+            m_s = fmaxf(mq[sq], mq[QW + sq]);
+            const float ma = mq[l32], mb = mq[QW + l32], mn = fmaxf(ma, mb);
+            const float corr = __builtin_amdgcn_exp2f(m_o - mn);
+            if (__builtin_amdgcn_ballot_w64(corr != 1.0f)) {
+#pragma unroll
+                for (int d = 0; d < 4; d++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++) o[d][i] *= corr;
+            }
+            m_o = mn;
+            float rs = 0.f;
+            const bool uneven = __builtin_amdgcn_ballot_w64(ma != mb) != 0;
+            const uint16_t *pr = p_lds + (qt * 32 + l32) * PRow + 8 * hh;
+            const uint16_t *vt = reinterpret_cast<const uint16_t *>(v_lds + buf * VBuf);
+#pragma unroll
+            for (int c = 0; c < KT / 16; c++) {
+                h8 p = *reinterpret_cast<const h8 *>(pr + 16 * c);
+                if (uneven) {
+                    const _Float16 f = (_Float16)__builtin_amdgcn_exp2f((c < KT / 32 ? ma : mb) - mn);
+                    p *= h8{f, f, f, f, f, f, f, f};
+                }
+#pragma unroll
+                for (int e = 0; e < 8; e += 2)
+                    rs = __builtin_amdgcn_fdot2(h2{p[e], p[e + 1]}, h2{(_Float16)1.f, (_Float16)1.f}, rs, false);
+#pragma unroll
+                for (int d = 0; d < 4; d++) {
+                    const h8 a = *reinterpret_cast<const h8 *>(
+                        vt + 2 * vt_at(128 * ds + 32 * d + l32, 0) + 16 * c + 8 * hh);
+                    o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, p, o[d], 0, 0, 0);
+                }
+            }
+            l_run = l_run * corr + rs;
+        }
+        __syncthreads();  // V(t), P and the maxima read; K(t+1), V(t+1) visible
+    }
+
+    const int my_q = tq0 + l32;
+    const float lt = l_run + __shfl_xor(l_run, 32, kWave);
+    if (my_q >= n_tok) return;
+    const float inv = lt > 0.f ? 1.0f / lt : 0.f;
+    typedef float f4_out __attribute__((ext_vector_type(4), aligned(4)));  // out is element-aligned
+    typedef _Float16 h4_out __attribute__((ext_vector_type(4), aligned(2)));
+    const size_t obase = ((size_t)my_q * n_q + qh) * HD + 128 * ds + 4 * hh;
+#pragma unroll
+    for (int d = 0; d < 4; d++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const size_t at = obase + 32 * d + 8 * g;
+            const f4_out v = {o[d][4 * g] * inv, o[d][4 * g + 1] * inv, o[d][4 * g + 2] * inv,
+                              o[d][4 * g + 3] * inv};
+            if constexpr (O16) {
+                const h4_out t = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+                *reinterpret_cast<h4_out *>(static_cast<uint16_t *>(outv) + at) = t;
+            } else {
+                *reinterpret_cast<f4_out *>(static_cast<float *>(outv) + at) = v;
+            }
+        }
+}
+
 }  // namespace
 
 int launch_attn_prefill_ipv(hipStream_t st, const float *q, const int8_t *kq, const uint16_t *ks,
@@ -1162,17 +1510,25 @@ int launch_attn_prefill_q8(hipStream_t st, const float *q, const int8_t *kq, con
         SGQ_CHECK(((uintptr_t)kq & 15) == 0 && ((uintptr_t)vq & 15) == 0,
                   "attn_prefill_q8: misaligned cache");
         const int qw = head_dim == 256 ? 128 : 64;  // queries per workgroup
-        const int qt = (n_tok + qw - 1) / qw;
+        const dim3 grid((n_tok + qw - 1) / qw, n_q);
         const uint32_t *no_step = nullptr;
         const uint16_t *no_qs = nullptr;
-        if (head_dim == 256)
-            hipLaunchKernelGGL((attn_prefill_wide_kernel<256, kPfQ8>), dim3(qt, n_q), dim3(512), 0,
-                               st, q, no_qs, src, out, n_tok, q0, no_step, n_q, n_kv, window, scale,
-                               qt);
-        else
-            hipLaunchKernelGGL((attn_prefill_wide_kernel<512, kPfQ8>), dim3(qt, n_q), dim3(512), 0,
-                               st, q, no_qs, src, out, n_tok, q0, no_step, n_q, n_kv, window, scale,
-                               qt);
+        // few keys in all: the wide kernel's shorter way through a single tile
+        // (head_dim 512, 20 / 100 / 200 / 400 keys 9.6 / 21.3 / 29.6 / 45.6 against
+        // 11.0 / 22.4 / 31.3 / 44.7 us; 256, 16 / 60 keys 7.7 / 13.4 against 8.7 /
+        // 12.7)
+        const bool few_keys = q0 + n_tok <= (head_dim == 256 ? 32 : 320);
+#define SGQ_PF_Q8(KERNEL, HD)                                                                    \
+    hipLaunchKernelGGL((KERNEL<HD, kPfQ8>), grid, dim3(512), 0, st, q, no_qs, src, out, n_tok, q0, \
+                       no_step, n_q, n_kv, window, scale, (int)grid.x)
+        if (head_dim == 256) {
+            if (few_keys) SGQ_PF_Q8(attn_prefill_wide_kernel, 256);
+            else SGQ_PF_Q8(attn_prefill_px_kernel, 256);
+        } else {
+            if (few_keys) SGQ_PF_Q8(attn_prefill_wide_kernel, 512);
+            else SGQ_PF_Q8(attn_prefill_px_kernel, 512);
+        }
+#undef SGQ_PF_Q8
         SGQ_HIP(hipGetLastError());
         return SGQ_OK;
     }
@@ -1217,19 +1573,19 @@ int launch_attn_prefill_pages(hipStream_t st, int fmt, const void *q, const uint
     const int qw = head_dim == 256 ? 128 : 64;  // queries per workgroup
     const int qt = (n_tok + qw - 1) / qw;
     const dim3 grid(qt, n_q);
-#define SGQ_PF_PAGES(HD, F)                                                                     \
-    hipLaunchKernelGGL((attn_prefill_wide_kernel<HD, F>), grid, dim3(512), 0, st, q, q_scales, src, \
-                       out, n_tok, 0, step, n_q, n_kv, window, scale, qt)
+#define SGQ_PF_PAGES(KERNEL, HD, F)                                                              \
+    hipLaunchKernelGGL((KERNEL<HD, F>), grid, dim3(512), 0, st, q, q_scales, src, out, n_tok, 0,     \
+                       step, n_q, n_kv, window, scale, qt)
     if (head_dim == 256) {
-        if (fmt == kPfQ8H) SGQ_PF_PAGES(256, kPfQ8H);
-        else if (fmt == kPfF16) SGQ_PF_PAGES(256, kPfF16);
-        else if (fmt == kPfIQ) SGQ_PF_PAGES(256, kPfIQ);
-        else SGQ_PF_PAGES(256, kPfIPV);
+        if (fmt == kPfQ8H) SGQ_PF_PAGES(attn_prefill_px_kernel, 256, kPfQ8H);
+        else if (fmt == kPfF16) SGQ_PF_PAGES(attn_prefill_px_kernel, 256, kPfF16);
+        else if (fmt == kPfIQ) SGQ_PF_PAGES(attn_prefill_wide_kernel, 256, kPfIQ);
+        else SGQ_PF_PAGES(attn_prefill_wide_kernel, 256, kPfIPV);
     } else {
-        if (fmt == kPfQ8H) SGQ_PF_PAGES(512, kPfQ8H);
-        else if (fmt == kPfF16) SGQ_PF_PAGES(512, kPfF16);
-        else if (fmt == kPfIQ) SGQ_PF_PAGES(512, kPfIQ);
-        else SGQ_PF_PAGES(512, kPfIPV);
+        if (fmt == kPfQ8H) SGQ_PF_PAGES(attn_prefill_px_kernel, 512, kPfQ8H);
+        else if (fmt == kPfF16) SGQ_PF_PAGES(attn_prefill_px_kernel, 512, kPfF16);
+        else if (fmt == kPfIQ) SGQ_PF_PAGES(attn_prefill_wide_kernel, 512, kPfIQ);
+        else SGQ_PF_PAGES(attn_prefill_wide_kernel, 512, kPfIPV);
     }
 #undef SGQ_PF_PAGES
     SGQ_HIP(hipGetLastError());

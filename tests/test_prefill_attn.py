@@ -142,3 +142,46 @@ def test_attn_prefill_wide_head_dims_match_oracle(ctx, oracle, hd, n_tok, q0, wi
         for h in range(n_q):
             want[i, h] = oracle.attention_head(q, kd, vd, i, h, n_q, n_kv, hd, scale, t0, p)
     _check(got, want, f"prefill hd={hd} n_tok={n_tok} q0={q0} w={window}")
+
+
+@pytest.mark.parametrize("hd,n_tok,q0,window", [
+    (256, 33, 0, 0), (256, 65, 0, 32), (256, 130, 100, 40), (256, 129, 63, 0), (256, 20, 500, 0),
+    (512, 64, 0, 0), (512, 70, 260, 0), (512, 33, 288, 0), (512, 40, 300, 33), (512, 16, 500, 100),
+    (512, 2, 319, 0)])
+@pytest.mark.parametrize("grow", [1.0, 4.0])
+def test_attn_prefill_wide_tile_edges(ctx, oracle, hd, n_tok, q0, window, grow):
+    """head_dim 256 / 512 around the key tiles (64 / 32 keys), the query tiles
+    and the switch of kernels at few keys, windows that leave whole key parts
+    of a tile masked; with grow > 1 the keys' magnitude rises by that factor
+    over the last third, so that reference maxima move inside the loop.  The
+    rounding of q to f16 moves a score by up to 2^-11 of its size, so the bar
+    of _check scales with the scores."""
+    n_q, n_kv = 4, 2
+    print(f"prefill edges hd={hd} n_tok={n_tok} q0={q0} window={window} grow={grow}", flush=True)
+    rng = oracle.Rng(0xED9E + hd + n_tok + q0 + window)
+    n_slots = q0 + n_tok
+    k = rng.f32_vec(n_slots * n_kv * hd).reshape(n_slots, -1)
+    k[2 * n_slots // 3:] *= np.float32(grow)
+    v = rng.f32_vec(n_slots * n_kv * hd)
+    ks, kq = oracle.quant_q8_0(k.reshape(-1))
+    vs, vq = oracle.quant_q8_0(v)
+    q = rng.f32_vec(n_tok * n_q * hd) * np.float32(2.0)
+    kd, vd = oracle.dequant_q8_0(ks, kq), oracle.dequant_q8_0(vs, vq)
+    scale = 1.0 / np.sqrt(hd)
+    buf = torch.full((n_tok * n_q * hd + 512,), float("nan"), dtype=torch.float32, device="cuda")
+    out = buf[256:-256]
+    ctx.attn_prefill_q8(dev(q), dev(kq), dev(ks), dev(vq), dev(vs), n_tok, q0, n_q, n_kv, out,
+                        window=window, scale=scale, head_dim=hd)
+    torch.cuda.synchronize()
+    all_ = host(buf)
+    assert np.isnan(all_[:256]).all() and np.isnan(all_[-256:]).all()
+    got = all_[256:-256].reshape(n_tok, n_q, hd)
+    want = np.empty_like(got)
+    for i in range(n_tok):
+        p = q0 + i
+        t0 = max(0, p + 1 - window) if window else 0
+        for h in range(n_q):
+            want[i, h] = oracle.attention_head(q, kd, vd, i, h, n_q, n_kv, hd, scale, t0, p)
+    f = 2.0 * grow
+    assert_close(got, want, f * 2e-3, f * 1e-3 * float(np.abs(want).max()), "prefill edges")
+    assert rel_err(got, want) <= f * 1e-3
