@@ -344,12 +344,13 @@ class AttnPrefillPages:
     window 1024: the ring holds the slots before the chunk, the chunk's own
     K/V come from its pages; groups [16, M, 1]).  One dispatch per step,
     replayed from a graph."""
-    kernel = "attn_prefill_wide_kernel"
 
     def __init__(self, ctx, torch, kind="global_flash_sp_iq", n_tok=4096):
         import struct
         import sgq
 
+        self.kernel = ("attn_prefill_px_kernel" if kind == "sliding_ring"
+                       else "attn_prefill_wide_kernel")
         self.ctx, self.kind, self.n_tok = ctx, kind, n_tok
         n_q = 32
         if kind == "sliding_ring":

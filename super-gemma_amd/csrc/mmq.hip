@@ -34,8 +34,8 @@
 //    1215-1221 -> 1146-1149 us there; K = 21504, M = 2048, split 4 666 -> 643;
 //    K = 5376, M = 512 172 -> 170.
 //  * Ragged tiles read clamped rows and run the same loop (they had a
-//    bounds-checked one: a 1500-token prompt of the released geometry
-//    15.3 -> 14.15 ms, M = 37, N = 8192 86 -> 81 us).
+//    bounds-checked one: 1500 tokens through six layers of the released
+//    geometry 15.3 -> 14.15 ms, M = 37, N = 8192 86 -> 81 us).
 //  * Tile order is XCD-aware: consecutive workgroup ids land on different
 //    XCDs (each with its own L2), so ids are remapped so that every XCD
 //    walks a contiguous range of N-tiles with all their M-tiles, and a
