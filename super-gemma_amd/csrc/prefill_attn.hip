@@ -13,9 +13,9 @@
 // the chunk's own pages (row = position - q0) when those are given, else
 // from the cache too.  They are dequantized to f16 as in the reference's
 // _sp_q8 variant; P is rounded to f16 for PV, as in the reference.  The
-// head_dim-256/512 kernel (attn_prefill_wide_kernel, below) also reads the
-// reference's other page formats: f16 K/V, int8 q with Q8_0 K, int8 V with
-// key-blocked scales (PfFmt).
+// head_dim-256/512 kernels (below) also read the reference's other page formats
+// (PfFmt): f16 K/V (attn_prefill_px_kernel), int8 q with Q8_0 K and int8 V with
+// key-blocked scales (attn_prefill_wide_kernel).
 //
 // Design (MFMA-bound: 4·hd flops per query-key pair against 2·hd·1 B of
 // K/V per key per query tile):
@@ -1101,13 +1101,14 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
         }
 }
 
-// The value of the lane 32 (16) away beside one's own, without the LDS trip of
-// a shuffle: {lanes 0-31 / even rows of 16, lanes 32-63 / odd rows} in both.
+// The larger of a lane's value and that of the lane 32 (16) away, without the
+// LDS trip of a shuffle.
 __device__ __forceinline__ float max_x32(float v) {
     const uint32_t b = __builtin_bit_cast(uint32_t, v);
     const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
     return fmaxf(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
 }
+
 __device__ __forceinline__ float max_x16(float v) {
     const uint32_t b = __builtin_bit_cast(uint32_t, v);
     const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
@@ -1122,28 +1123,32 @@ __device__ __forceinline__ float max_x16(float v) {
 //                           (v_mfma_f32_32x32x16_f16);
 //   head_dim 512 (KT = 32): wave ds takes 16 keys × 16 queries
 //                           (v_mfma_f32_16x16x32_f16).
-// Each wave writes its P as f16 and the reference max it used to LDS; after
-// the barrier every wave reads the tile's whole P as the B operand of
-// Oᵀ = Vᵀ·Pᵀ for its own 128 dims.  A reference is the query's maximum over the
-// first tile (exchanged there, one more barrier) and moves rarely (lazily, by
-// more than 2^8) and by whole powers of two, so that bringing the parts of P to
-// their common one is exact.  The denominator sums P as rounded to f16, as the
-// numerator does.
-// Per tile: scores, P out → barrier → PV(t), K(t+1) and V(t+1) staged from
-// registers (V double-buffered), quants of t+2 issued → barrier.
-// It replaces attn_prefill_wide_kernel, whose D waves each compute partial
-// scores over 128 dims, exchange them as f32 and repeat the softmax, for the
-// f16 and Q8_0 formats (us, before -> after; kv heads 16 / 4): head_dim 256,
-// Q8_0, 1024 window, 4096 queries 401 -> 306, 1111 queries from 2003 196 ->
-// 155; f16 ring, 512 queries from 1777 84 -> 72; head_dim 512, Q8_0, causal,
-// 2000 queries 406 -> 365, 20 queries from 3000 259 -> 195; f16, 1024 queries
-// from 1000 290 -> 257.  What bounds it: waits between dependent LDS reads and
-// MFMAs (two waves per SIMD), then the dequant's VALU.  Two forms with fewer
-// waves per score measured slower: 256 dims per wave (spills; f16 ring of 2048
-// queries 199 against 145), all dims in one wave per SIMD with Oᵀ in
-// accumulation registers (1029 for the 1111 queries).  Int8 q stays with the
-// wide kernel: here its block scales spill (322 -> 1020 for 1024 queries from
-// 1024).
+// Each wave writes its P to LDS; after the barrier every wave reads the tile's
+// whole P as the B operand of Oᵀ = Vᵀ·Pᵀ for its own 128 dims.  At head_dim 256
+// a wave has 32 keys of a query, rounds them to f16 and writes their fp32 sum
+// beside them; at 512 P goes through LDS in fp32, and the readers sum and round.
+// The numerics are attn_prefill_wide_kernel's, bit for bit: scores, fp32
+// denominators and outputs are summed in its order, under one reference maximum
+// per query and 32 keys, which moves when the maximum has passed it by 2^8.  P is
+// written for the reference as it stands.  A wave that finds that a reference has
+// to move (in the first tile, then rarely) raises a flag, on which the workgroup
+// takes one more barrier to agree on the references and write P again.
+// Per tile: scores, P out → barrier → K(t+1) and V(t+1) staged from registers
+// (V double-buffered), quants of t+2 issued, PV(t) → barrier.
+// Against attn_prefill_wide_kernel, whose D waves each compute partial scores
+// over 128 dims, exchange them as fp32 and repeat the softmax (us, wide -> here;
+// kv heads 16 / 4): head_dim 256, Q8_0, 1024 window, 4096 queries 401 -> 311,
+// 1111 queries from 2003 195 -> 156; f16 ring, 512 queries from 1777 84 -> 72;
+// head_dim 512, Q8_0, causal, 2000 queries 404 -> 393, 20 queries from 3000 260
+// -> 201; f16, 1024 queries from 1000 290 -> 276.  What bounds it: waits between
+// dependent LDS reads and MFMAs (two waves per SIMD), then the dequant's VALU.
+// Other forms: denominators from P as rounded to f16, with a reference per key
+// part (2000 queries of 512: 364, but fewer bits in the sums); 256 dims per wave
+// (spills; f16 ring of 2048 queries 199 against 145); all dims in one wave per
+// SIMD with Oᵀ in accumulation registers (1029 for the 1111 queries); the wide
+// kernel's scores with only the softmax cut (2000 queries of 512: 429).  Int8 q
+// stays with the wide kernel: here its block scales spill (322 -> 1020 for 1024
+// queries from 1024).
 template <int HD, int FMT>
 __global__ __launch_bounds__(512, 2) void attn_prefill_px_kernel(
     const void *__restrict__ qv, const uint16_t *__restrict__ q_scales, KvSource src,
@@ -1154,21 +1159,24 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_px_kernel(
     constexpr bool S32 = HD == 256;           // scores as a 32×32 tile (else 16×16)
     constexpr int D = HD / 128;               // waves per query tile
     constexpr int QW = 32 * (8 / D);          // queries per workgroup
-    constexpr int KT = S32 ? 64 : 32;         // keys per tile
+    constexpr int KT = S32 ? 64 : 32, G = KT / 32;  // keys per tile, 32 to a reference
     constexpr int NB = HD / 32, NP = KT / 2, CW = 16;
     static_assert(NP * (HD / CW) == 512, "one staging item per thread");
     constexpr int KRowB = (HD + 8) * 2;       // bytes per K row (f16) in LDS
     constexpr int VS = NP + 4;                // Vᵀ row, dwords (16-byte reads, 4 banks apart)
     constexpr int VPad = S32 ? 0 : 16;        // dwords per 16 rows: the staging writes of a wave
     constexpr int VBuf = HD * VS + (HD / 16) * VPad;
-    constexpr int PRow = KT + 8;              // P row (halves): [query][key]
-    constexpr int kKBytes = KT * KRowB, kVBytes = 2 * VBuf * 4, kPBytes = QW * PRow * 2;
-    constexpr int kMBytes = 4 * QW * 4;       // [key part][query]: reference maxima, first maxima
+    constexpr int PRow = KT + 8;              // P row (halves, S32): [query][key, in operand order]
+    constexpr int kPBytes = S32 ? QW * PRow * 2 : QW * 32 * 4;
+    constexpr int kKBytes = KT * KRowB, kVBytes = 2 * VBuf * 4;
+    constexpr int kMBytes = 4 * QW * 4;       // [key part][query]: maxima, then (S32) sums of P
     __shared__ __align__(16) uint8_t lds[kKBytes + kVBytes + kPBytes + kMBytes];
+    __shared__ uint32_t moved[2];             // a reference moves in this tile / the next
     uint8_t *const k_lds = lds;
     uint32_t *const v_lds = reinterpret_cast<uint32_t *>(lds + kKBytes);
     uint16_t *const p_lds = reinterpret_cast<uint16_t *>(lds + kKBytes + kVBytes);
     float *const m_lds = reinterpret_cast<float *>(lds + kKBytes + kVBytes + kPBytes);
+    float *const l_lds = m_lds + 2 * QW;
     auto vt_at = [](int row, int col) { return row * VS + (row >> 4) * VPad + col; };
 
     int bx = (int)blockIdx.x, by = (int)blockIdx.y;
@@ -1184,36 +1192,41 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_px_kernel(
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int qt = wave / D, ds = wave % D;
     const int l32 = lane & 31, hh = lane >> 5;
-    // this wave's scores: key part kp (of 2), and this lane's score query sq
-    // (of the tile's 32); A / B operand row within the part and K quarter
+    const int tq0 = tile * QW + qt * 32;     // the query tile's first query
+    // this wave's scores: key part kp (of 2) for query sq of the tile, A / B
+    // operand row orow within the part and quarter (S32: half) okq of the K slots
     const int kp = S32 ? ds : ds >> 1;
     const int sq = S32 ? l32 : 16 * (ds & 1) + (lane & 15);
     const int orow = S32 ? l32 : lane & 15, okq = S32 ? hh : lane >> 4;
-    const int tq0 = tile * QW + qt * 32;     // the query tile's first query
     const int my_s = tq0 + sq;
     const bool s_valid = my_s < n_tok;
-    const int sp = q0 + my_s;                // the score query's position
+    const int sp = q0 + my_s;
 
     const float qscale = scale * 1.44269504088896341f;
-    constexpr int NC = S32 ? HD / 16 : HD / 32;  // MFMA steps over the dims
+    // MFMA steps over the dims: 16 (32) each.  The first dim of step c: the two
+    // chains of 128 dims take 16 dims in turn, and a K-32 step, which rounds as
+    // two K-16 steps do, two of a chain's.
+    constexpr int NC = S32 ? HD / 16 : HD / 32;
+    const int od = S32 ? 8 * hh : 32 * (okq >> 1) + 8 * (okq & 1);
+    auto dim_of = [](int c) { return S32 ? 16 * c : 64 * (c >> 1) + 16 * (c & 1); };
     h8 qb[NC];
     {
         const size_t row = (size_t)(s_valid ? my_s : 0) * n_q + qh;
         if constexpr (QF32) {
-            const float *qr = static_cast<const float *>(qv) + row * HD + 8 * okq;
+            const float *qr = static_cast<const float *>(qv) + row * HD + od;
 #pragma unroll
             for (int c = 0; c < NC; c++) {
-                const float4 x = *reinterpret_cast<const float4 *>(qr + (HD / NC) * c);
-                const float4 y = *reinterpret_cast<const float4 *>(qr + (HD / NC) * c + 4);
+                const float4 x = *reinterpret_cast<const float4 *>(qr + dim_of(c));
+                const float4 y = *reinterpret_cast<const float4 *>(qr + dim_of(c) + 4);
                 const float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
 #pragma unroll
                 for (int e = 0; e < 8; e++) qb[c][e] = (_Float16)(s_valid ? v[e] * qscale : 0.f);
             }
         } else {
-            const uint16_t *qr = static_cast<const uint16_t *>(qv) + row * HD + 8 * okq;
+            const uint16_t *qr = static_cast<const uint16_t *>(qv) + row * HD + od;
 #pragma unroll
             for (int c = 0; c < NC; c++) {
-                const h8 t = __builtin_bit_cast(h8, *reinterpret_cast<const uint4 *>(qr + (HD / NC) * c));
+                const h8 t = __builtin_bit_cast(h8, *reinterpret_cast<const uint4 *>(qr + dim_of(c)));
                 qb[c] = s_valid ? t : h8{};
             }
         }
@@ -1223,8 +1236,8 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_px_kernel(
     for (int d = 0; d < 4; d++)
 #pragma unroll
         for (int i = 0; i < 16; i++) o[d][i] = 0.f;
-    // reference maxima of the score query and of the output query (l32), and
-    // the output query's sum over this half's keys
+    // references of the score query and of the output query (l32), which has
+    // the denominator
     float m_s = kNegBig, m_o = kNegBig, l_run = 0.f;
 
     const int qpos_lo = q0 + tile * QW;
@@ -1235,6 +1248,9 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_px_kernel(
     // staging item of this thread: keys 2·pair, 2·pair + 1 of the tile, dims
     // dim0 .. +15
     const int pair = tid % NP, dim0 = CW * (tid / NP), blk = dim0 >> 5;
+    // its Vᵀ column: of 16 keys, operand half h holds 4h .. +3 and 8 + 4h .. +3,
+    // the keys whose scores the lanes of half h hold
+    const int vcol = (pair & ~6) | (pair & 2) << 1 | (pair & 4) >> 1;
     constexpr int EK = F16 ? 2 : 1, EV = F16 ? 2 : 1;  // bytes per K / V element
     const char *const kq_c = sgpr_ptr(reinterpret_cast<const char *>(src.kq));
     const char *const vq_c = sgpr_ptr(reinterpret_cast<const char *>(src.vq));
@@ -1317,35 +1333,67 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_px_kernel(
             }
         }
 #pragma unroll
-        for (int j = 0; j < CW; j++) vt[vt_at(dim0 + j, pair)] = vpk[j];
+        for (int j = 0; j < CW; j++) vt[vt_at(dim0 + j, vcol)] = vpk[j];
     };
 
     constexpr int NS = S32 ? 16 : 4;  // scores per lane
     typedef float sv_t __attribute__((ext_vector_type(NS)));
     // key of score i within the tile
     auto skey = [&](int i) { return S32 ? 32 * kp + 8 * (i / 4) + 4 * hh + (i % 4) : 16 * kp + 4 * okq + i; };
+    // this wave's scores: per 128 dims two chains, the sums in order
     auto scores = [&]() {
-        const uint8_t *kr = k_lds + ((S32 ? 32 : 16) * kp + orow) * KRowB;
-        sv_t s0, s1;
+        const uint8_t *kr = k_lds + ((S32 ? 32 : 16) * kp + orow) * KRowB + 2 * od;
+        sv_t s;
 #pragma unroll
-        for (int i = 0; i < NS; i++) s0[i] = s1[i] = 0.f;
+        for (int g = 0; g < D; g++) {
+            sv_t s0, s1;
 #pragma unroll
-        for (int c = 0; c < NC; c += 2) {
-            const h8 a0 = *reinterpret_cast<const h8 *>(kr + 2 * ((HD / NC) * c + 8 * okq));
-            const h8 a1 = *reinterpret_cast<const h8 *>(kr + 2 * ((HD / NC) * (c + 1) + 8 * okq));
-            if constexpr (S32) {
-                s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, qb[c], s0, 0, 0, 0);
-                s1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, qb[c + 1], s1, 0, 0, 0);
-            } else {
-                s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, qb[c], s0, 0, 0, 0);
-                s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, qb[c + 1], s1, 0, 0, 0);
+            for (int i = 0; i < NS; i++) s0[i] = s1[i] = 0.f;
+#pragma unroll
+            for (int c = NC / D * g; c < NC / D * (g + 1); c += 2) {
+                const h8 a0 = *reinterpret_cast<const h8 *>(kr + 2 * dim_of(c));
+                const h8 a1 = *reinterpret_cast<const h8 *>(kr + 2 * dim_of(c + 1));
+                if constexpr (S32) {
+                    s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, qb[c], s0, 0, 0, 0);
+                    s1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, qb[c + 1], s1, 0, 0, 0);
+                } else {
+                    s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, qb[c], s0, 0, 0, 0);
+                    s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, qb[c + 1], s1, 0, 0, 0);
+                }
             }
-        }
 #pragma unroll
-        for (int i = 0; i < NS; i++) s0[i] += s1[i];
-        return s0;
+            for (int i = 0; i < NS; i++) s[i] = g ? s[i] + (s0[i] + s1[i]) : s0[i] + s1[i];
+        }
+        return s;
+    };
+    // P of this wave's scores for the reference m.  S32: f16, in operand order,
+    // beside the sum over the 32 keys; else fp32, as the lanes of the output
+    // queries sum and round them (float4 [8 keys][lane])
+    auto put_p = [&](const sv_t &s, bool full, float m) {
+        float p[NS];
+#pragma unroll
+        for (int i = 0; i < NS; i++)
+            p[i] = full || s[i] > kNegBig ? __builtin_amdgcn_exp2f(s[i] - m) : 0.f;
+        if constexpr (S32) {
+            float rs = 0.f;
+            h8 pb[2];
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                rs += p[i];
+                pb[i / 8][i % 8] = (_Float16)p[i];
+            }
+            rs += __shfl_xor(rs, 32, kWave);
+            uint16_t *pr = p_lds + (qt * 32 + l32) * PRow + 32 * kp + 8 * hh;
+            *reinterpret_cast<h8 *>(pr) = pb[0];
+            *reinterpret_cast<h8 *>(pr + 16) = pb[1];
+            if (hh == 0) l_lds[kp * QW + qt * 32 + l32] = rs;
+        } else {
+            reinterpret_cast<float4 *>(p_lds)[(qt * 4 + 2 * kp + (okq >> 1)) * 64 + 32 * (okq & 1) + sq] =
+                make_float4(p[0], p[1], p[2], p[3]);
+        }
     };
 
+    if (tid < 2) moved[tid] = 0u;
     fetch(k_lo);
     stage(k_lo, 0);
     if (k_lo + KT <= k_hi) fetch(k_lo + KT);
@@ -1355,9 +1403,9 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_px_kernel(
     for (int kl = k_lo; kl <= k_hi; kl += KT, buf ^= 1) {
         // some query of the tile sees some key (the same in its D waves)
         const bool live = tq_lo <= k_hi && kl <= tq_hi && (window <= 0 || kl + KT - 1 > tq_lo - window);
-        float m_part = m_s, mx = kNegBig;
+        const int kb = S32 ? kl + 32 * kp : kl;
+        const bool full = kb + 31 <= tq_lo && (window <= 0 || kb > tq_lo + 31 - window);
         sv_t s;
-        const bool full = kl + KT - 1 <= tq_lo && (window <= 0 || kl > tq_lo + 31 - window);
         if (live) {
             s = scores();
             if constexpr (!QF32)
@@ -1371,82 +1419,102 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_px_kernel(
                     s[i] = ok ? s[i] : kNegBig;
                 }
             }
-            mx = s[0];
+            float mx = s[0];
 #pragma unroll
             for (int i = 1; i < NS; i++) mx = fmaxf(mx, s[i]);
             if constexpr (!S32) mx = max_x16(mx);
             mx = max_x32(mx);
+            if (okq == 0) m_lds[kp * QW + qt * 32 + sq] = mx;
+            if (__builtin_amdgcn_ballot_w64(mx > m_s + 8.0f) && lane == 0) moved[buf] = 1u;
+            put_p(s, full, m_s);
         }
-        if (kl == k_lo) {  // the first references, common to the parts: one more barrier
-            float *m0 = m_lds + 2 * QW + qt * 32 + sq;
-            if (live && (S32 ? hh == 0 : okq == 0)) m0[kp * QW] = mx;
-            __syncthreads();
-            if (live) m_part = fmaxf(m0[0], m0[QW]);
-        } else if (mx > m_s + 8.0f) {
-            m_part = m_s > kNegBig ? m_s + __builtin_ceilf(mx - m_s) : __builtin_ceilf(mx);
-        }
-        if (live) {
-            uint32_t pw[NS / 2];
-#pragma unroll
-            for (int i = 0; i < NS; i += 2) {
-                const float p0 = full || s[i] > kNegBig ? __builtin_amdgcn_exp2f(s[i] - m_part) : 0.f;
-                const float p1 = full || s[i + 1] > kNegBig ? __builtin_amdgcn_exp2f(s[i + 1] - m_part) : 0.f;
-                const h2 t = {(_Float16)p0, (_Float16)p1};
-                pw[i / 2] = __builtin_bit_cast(uint32_t, t);
+        __syncthreads();  // P, its sums and the maxima visible; K fully read
+        const uint32_t flag = moved[buf];
+        if constexpr (!S32)  // staged while the flag is on its way
+            if (kl + KT <= k_hi) {
+                stage(kl + KT, buf ^ 1);
+                if (kl + 2 * KT <= k_hi) fetch(kl + 2 * KT);
             }
-            uint16_t *pr = p_lds + (qt * 32 + sq) * PRow;
+        float corr[G];
 #pragma unroll
-            for (int j = 0; j < NS / 4; j++)
-                *reinterpret_cast<uint2 *>(pr + skey(4 * j)) = make_uint2(pw[2 * j], pw[2 * j + 1]);
-            if (S32 ? hh == 0 : okq == 0) m_lds[kp * QW + qt * 32 + sq] = m_part;
-        }
-        __syncthreads();  // P and the maxima visible; K fully read
-        if (kl + KT <= k_hi) {
-            stage(kl + KT, buf ^ 1);
-            if (kl + 2 * KT <= k_hi) fetch(kl + 2 * KT);
-        }
-        if (live) {
-            const float *mq = m_lds + qt * 32;
-            m_s = fmaxf(mq[sq], mq[QW + sq]);
-            const float ma = mq[l32], mb = mq[QW + l32], mn = fmaxf(ma, mb);
-            const float corr = __builtin_amdgcn_exp2f(m_o - mn);
-            if (__builtin_amdgcn_ballot_w64(corr != 1.0f)) {
+        for (int g = 0; g < G; g++) corr[g] = 1.0f;
+        const bool move = __builtin_amdgcn_readfirstlane(flag) != 0;
+        if (tid == 0) moved[buf ^ 1] = 0u;
+        if (move) {  // the same in every wave
+            if (live) {
+                // the reference after 32 keys: their maximum, if it has passed the
+                // reference before them by 2^8
+                auto next = [&](float m, int q, int g) {
+                    const float *mq = m_lds + qt * 32 + q;
+                    const float mx = S32 ? mq[g * QW] : fmaxf(mq[0], mq[QW]);
+                    return mx > m + 8.0f ? mx : m;
+                };
+                float mine = m_s;
 #pragma unroll
-                for (int d = 0; d < 4; d++)
-#pragma unroll
-                    for (int i = 0; i < 16; i++) o[d][i] *= corr;
+                for (int g = 0; g < G; g++) {
+                    m_s = next(m_s, sq, g);
+                    if (!S32 || g <= kp) mine = m_s;
+                    const float to = next(m_o, l32, g);
+                    corr[g] = __builtin_amdgcn_exp2f(m_o - to);
+                    m_o = to;
+                }
+                put_p(s, full, mine);
             }
-            m_o = mn;
-            float rs = 0.f;
-            const bool uneven = __builtin_amdgcn_ballot_w64(ma != mb) != 0;
-            const uint16_t *pr = p_lds + (qt * 32 + l32) * PRow + 8 * hh;
-            const uint16_t *vt = reinterpret_cast<const uint16_t *>(v_lds + buf * VBuf);
+            __syncthreads();  // P for the references agreed on
+        }
+        if constexpr (S32)
+            if (kl + KT <= k_hi) {
+                stage(kl + KT, buf ^ 1);
+                if (kl + 2 * KT <= k_hi) fetch(kl + 2 * KT);
+            }
+        if (live) {
+            const uint16_t *vt = reinterpret_cast<const uint16_t *>(v_lds + buf * VBuf) + 8 * hh;
 #pragma unroll
-            for (int c = 0; c < KT / 16; c++) {
-                h8 p = *reinterpret_cast<const h8 *>(pr + 16 * c);
-                if (uneven) {
-                    const _Float16 f = (_Float16)__builtin_amdgcn_exp2f((c < KT / 32 ? ma : mb) - mn);
-                    p *= h8{f, f, f, f, f, f, f, f};
+            for (int g = 0; g < G; g++) {
+                h8 pb[2];
+                float rs;
+                if constexpr (S32) {
+                    const uint16_t *pr = p_lds + (qt * 32 + l32) * PRow + 32 * g + 8 * hh;
+                    pb[0] = *reinterpret_cast<const h8 *>(pr);
+                    pb[1] = *reinterpret_cast<const h8 *>(pr + 16);
+                    rs = l_lds[g * QW + qt * 32 + l32];
+                } else {
+                    rs = 0.f;
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const float4 v = reinterpret_cast<const float4 *>(p_lds)[(qt * 4 + j) * 64 + lane];
+                        const float pv[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            rs += pv[e];
+                            pb[j / 2][4 * (j & 1) + e] = (_Float16)pv[e];
+                        }
+                    }
+                    rs += __shfl_xor(rs, 32, kWave);
+                }
+                l_run = l_run * corr[g] + rs;
+                if (move && __builtin_amdgcn_ballot_w64(corr[g] != 1.0f)) {
+#pragma unroll
+                    for (int d = 0; d < 4; d++)
+#pragma unroll
+                        for (int i = 0; i < 16; i++) o[d][i] *= corr[g];
                 }
 #pragma unroll
-                for (int e = 0; e < 8; e += 2)
-                    rs = __builtin_amdgcn_fdot2(h2{p[e], p[e + 1]}, h2{(_Float16)1.f, (_Float16)1.f}, rs, false);
+                for (int c = 0; c < 2; c++)
 #pragma unroll
-                for (int d = 0; d < 4; d++) {
-                    const h8 a = *reinterpret_cast<const h8 *>(
-                        vt + 2 * vt_at(128 * ds + 32 * d + l32, 0) + 16 * c + 8 * hh);
-                    o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, p, o[d], 0, 0, 0);
-                }
+                    for (int d = 0; d < 4; d++) {
+                        const h8 a = *reinterpret_cast<const h8 *>(
+                            vt + 2 * vt_at(128 * ds + 32 * d + l32, 0) + 32 * g + 16 * c);
+                        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pb[c], o[d], 0, 0, 0);
+                    }
             }
-            l_run = l_run * corr + rs;
         }
-        __syncthreads();  // V(t), P and the maxima read; K(t+1), V(t+1) visible
+        __syncthreads();  // V(t), P and its sums read; K(t+1), V(t+1) visible
     }
 
     const int my_q = tq0 + l32;
-    const float lt = l_run + __shfl_xor(l_run, 32, kWave);
     if (my_q >= n_tok) return;
-    const float inv = lt > 0.f ? 1.0f / lt : 0.f;
+    const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
     typedef float f4_out __attribute__((ext_vector_type(4), aligned(4)));  // out is element-aligned
     typedef _Float16 h4_out __attribute__((ext_vector_type(4), aligned(2)));
     const size_t obase = ((size_t)my_q * n_q + qh) * HD + 128 * ds + 4 * hh;
@@ -1518,11 +1586,14 @@ int launch_attn_prefill_q8(hipStream_t st, const float *q, const int8_t *kq, con
         const dim3 grid((n_tok + qw - 1) / qw, n_q);
         const uint32_t *no_step = nullptr;
         const uint16_t *no_qs = nullptr;
-        // few keys in all: the wide kernel's shorter way through a single tile
-        // (head_dim 512, 20 / 100 / 200 / 400 keys 9.6 / 21.3 / 29.6 / 45.6 against
-        // 11.0 / 22.4 / 31.3 / 44.7 us; 256, 16 / 60 keys 7.7 / 13.4 against 8.7 /
-        // 12.7)
-        const bool few_keys = q0 + n_tok <= (head_dim == 256 ? 32 : 320);
+        // Few keys in all: the wide kernel's shorter way through a single tile, with
+        // the same bits.  us, wide / px: head_dim 256, 16 / 30 / 40 keys 8.0 / 8.9 /
+        // 12.0 against 9.2 / 10.2 / 11.4; 512, as many queries as keys, 20 / 100 /
+        // 320 / 500 / 700: 9.6 / 21.0 / 40.1 / 56.4 / 72.9 against 11.1 / 23.2 /
+        // 42.1 / 56.7 / 72.7; 20 queries (px: a query tile without queries rests),
+        // 100 / 200 / 320 keys 18.4 / 26.4 / 33.4 against 18.3 / 24.2 / 29.7.
+        const int n_keys = q0 + n_tok;
+        const bool few_keys = n_keys <= (head_dim == 256 ? 32 : n_tok > 32 ? 512 : 96);
 #define SGQ_PF_Q8(KERNEL, HD)                                                                    \
     hipLaunchKernelGGL((KERNEL<HD, kPfQ8>), grid, dim3(512), 0, st, q, no_qs, src, out, n_tok, q0, \
                        no_step, n_q, n_kv, window, scale, (int)grid.x)

@@ -185,3 +185,59 @@ def test_attn_prefill_wide_tile_edges(ctx, oracle, hd, n_tok, q0, window, grow):
     f = 2.0 * grow
     assert_close(got, want, f * 2e-3, f * 1e-3 * float(np.abs(want).max()), "prefill edges")
     assert rel_err(got, want) <= f * 1e-3
+
+
+@pytest.mark.parametrize("hd,n_kv", [(256, 2), (512, 1)])
+def test_attn_prefill_denominator_keeps_small_probabilities(ctx, oracle, hd, n_kv):
+    """A dominating first key (weight 1, V = 127/128) before some 4000 keys of weight
+    2^-25.3 each (V = 0): P is rounded to f16, where they are zero, but the
+    denominator is the fp32 sum of the unrounded P, so the output is
+    V / (1 + n·2^-25.3), 1e-4 below V.  Bar 2e-5: the running fp32 sum may lose
+    half an ulp of 1 per 32 keys (125 · 6e-8), and a weight off by q's f16
+    rounding (25.3 · 2^-12 of its exponent) moves the result by 4e-7; K and V
+    are f16 numbers."""
+    n_q, n_tok, q0 = 2 * n_kv, 40, 4000
+    n_slots = q0 + n_tok
+    gap = 25.3 * np.log(2.0)  # between the first key's score and the others'
+    scale = 1.0 / np.sqrt(hd)
+    print(f"prefill denominator hd={hd}", flush=True)
+    k = np.zeros((n_slots, n_kv, hd), np.float32)
+    k[0] = 127.0 / 64.0  # 127 quants of 2^-6
+    q = np.full((n_tok, n_q, hd), gap / (hd * scale * k[0, 0, 0]), np.float32)
+    v = np.zeros_like(k)
+    v[0] = 127.0 / 128.0
+    ks, kq = oracle.quant_q8_0(k.reshape(-1))
+    vs, vq = oracle.quant_q8_0(v.reshape(-1))
+    out = empty(n_tok * n_q * hd, torch.float32)
+    ctx.attn_prefill_q8(dev(q.reshape(-1)), dev(kq), dev(ks), dev(vq), dev(vs), n_tok, q0, n_q, n_kv,
+                        out, scale=scale, head_dim=hd)
+    torch.cuda.synchronize()
+    got = host(out).reshape(n_tok, -1).astype(np.float64)
+    assert oracle.dequant_q8_0(ks, kq)[0] == k[0, 0, 0] and oracle.dequant_q8_0(vs, vq)[0] == v[0, 0, 0]
+    # besides the first, query i sees q0 + i keys
+    want = v[0, 0, 0] / (1.0 + np.exp(-gap) * np.arange(q0, q0 + n_tok))
+    assert np.abs(got / want[:, None] - 1.0).max() <= 2e-5
+
+
+@pytest.mark.parametrize("hd,q0,short,long_", [
+    (256, 0, 20, 150), (256, 0, 32, 33), (512, 0, 60, 600), (512, 60, 20, 470), (512, 0, 512, 513)])
+@pytest.mark.parametrize("grow", [1.0, 4.0])
+def test_attn_prefill_rows_do_not_depend_on_the_chunk(ctx, oracle, hd, q0, short, long_, grow):
+    """Few keys take another kernel than many: the rows that a short and a long
+    chunk share have the same bits, also where the references move."""
+    n_q, n_kv = 4, 2
+    print(f"prefill chunks hd={hd} q0={q0} {short}/{long_} grow={grow}", flush=True)
+    rng = oracle.Rng(0xB175 + hd + q0 + long_)
+    k = rng.f32_vec((q0 + long_) * n_kv * hd).reshape(q0 + long_, -1)
+    k[(q0 + short) // 3:] *= np.float32(grow)
+    ks, kq = oracle.quant_q8_0(k.reshape(-1))
+    vs, vq = oracle.quant_q8_0(rng.f32_vec(k.size))
+    q = rng.f32_vec(long_ * n_q * hd) * np.float32(2.0)
+    got = []
+    for n in (short, long_):
+        out = empty(n * n_q * hd, torch.float32)
+        ctx.attn_prefill_q8(dev(q[:n * n_q * hd]), dev(kq), dev(ks), dev(vq), dev(vs), n, q0, n_q, n_kv,
+                            out, scale=1.0 / np.sqrt(hd), head_dim=hd)
+        torch.cuda.synchronize()
+        got.append(host(out, np.uint32).reshape(n, -1)[:short])
+    assert np.array_equal(got[0], got[1])
