@@ -1263,22 +1263,16 @@ int sgq_model_fill_cache(sgq_model *m, uint32_t n_tokens, uint64_t seed) {
 namespace {
 
 // Split-K factor for an MMQ of m×n×k: enough (tile, split) work items to fill
-// the chip's workgroup slots, at least 16 blocks of K per split.  512 128×128
-// workgroups are resident; doubling stops at 1.5 rounds of them, because from
-// there a split's extra partial sums and half-empty second round cost more
-// than it fills.  With `<= 1024` the rule went one doubling too far for these
-// (us at splits 1/2/4/8):
-//   m=100  n=16384 k=5376   48.8/49.5/44.3/56.2   (128 tiles: took 8, now 4)
-//   m=300  n=5376  k=8192    121/69/59/65         (126 tiles: took 8, now 4)
-//   m=300  n=5376  k=21504   311/164/134.5/140    (126 tiles: took 8, now 4)
-//   m=700  n=5376  k=8192    122/104.5/114.6/131  (252 tiles: took 4, now 2)
-//   m=700  n=5376  k=21504   313/253/257/269      (252 tiles: took 4, now 2)
-//   m=1500 n=5376  k=8192    181/200/215/245      (504 tiles: took 2, now 1)
-//   m=1500 n=5376  k=21504   480/488/495/530      (504 tiles: took 2, now 1)
+// the chip's workgroup slots, at least 16 blocks of K per split.  Stopping at 768
+// items (1.5 rounds of the 512 resident workgroups) was measured 0.5-5% faster for
+// whole prompts (released geometry, six layers: 300 tokens 4.62 -> 4.40 ms, 700
+// 7.62 -> 7.59, 1500 14.10 -> 14.01), but it groups the partial sums differently,
+// and a last-place change there moves single Q8_0 quants of the layers behind:
+// the logits of 1500 tokens by 3-4e-3.
 uint32_t mmq_split(uint32_t m, uint32_t n, uint32_t k) {
     const uint64_t tiles = (uint64_t)((m + 127) / 128) * ((n + 127) / 128);
     uint32_t split = 1;
-    while (split < 8 && tiles * split * 2 <= 768 && (k / 32) / (split * 2) >= 16) split *= 2;
+    while (split < 8 && tiles * split * 2 <= 1024 && (k / 32) / (split * 2) >= 16) split *= 2;
     return split;
 }
 constexpr size_t kPfPartialFloats = 1024ull * 128 * 128;  // >= split·m·n for every choice above
