@@ -578,6 +578,11 @@ __global__ __launch_bounds__(W * 64, 2) void mmq_skinny_kernel(
         for (int i = 0; i < 4 * TM; i++) *reinterpret_cast<v4i *>(wa + i * 1024) = ga[i];
 #pragma unroll
         for (int i = 0; i < 9; i++) lb[i * 64 + lane] = gb[i];
+        // the wave's other lanes read these: ordered for the compiler (LDS
+        // operations of one wave complete in order)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         uint32_t sa[TM][2];
 #pragma unroll
         for (int i = 0; i < TM; i++) {
@@ -614,6 +619,10 @@ __global__ __launch_bounds__(W * 64, 2) void mmq_skinny_kernel(
                 }
             }
         }
+        // this step's reads before the next step's stores
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
     __syncthreads();  // every wave is done with its tile
     float(*red)[TM * 16 * 64] = reinterpret_cast<float(*)[TM * 16 * 64]>(lds);
