@@ -60,10 +60,12 @@ def test_mmq_small_full_check(ctx, oracle, m, k, n):
     (1, 64, 1, 1), (33, 64, 127, 1), (127, 192, 129, 1), (129, 448, 256, 1), (256, 1216, 128, 1),
     (128, 320, 131, 1), (65, 1088, 132, 4), (300, 2112, 260, 8),
     (16, 128, 31, 1), (31, 2112, 96, 8), (32, 64, 33, 1), (64, 1088, 65, 2), (96, 192, 64, 1),
-    (97, 576, 37, 1), (2, 192, 16390, 1), (40, 128, 16385, 1)])
+    (97, 576, 37, 1), (2, 192, 16390, 1), (40, 128, 16385, 1), (100, 128, 16390, 1),
+    (129, 64, 127, 1), (132, 64, 130, 8), (132, 192, 130, 2), (132, 192, 130, 4)])
 def test_mmq_tile_and_k_edges(ctx, oracle, m, k, n, split):
     """Rows and columns around the tile edges with a K that ends in two
-    blocks (k % 128 == 64, one stage at K = 64), whole and split over K:
+    blocks (k % 128 == 64, one stage at K = 64), whole and split over K, also
+    into more parts than K has stages and with a last part of two blocks:
     every element against the oracle, the operands at the very end of their
     buffers and the output's surroundings untouched.  Up to 64 rows (128
     unsplit) the few-rows kernel answers: its row tiles' edges, K ranges
@@ -114,6 +116,87 @@ def test_mmq_integer_tile_is_exact(ctx, oracle):
     ctx.gemm_q4_0_q8(dev(w.reshape(-1)), dev(a.astype(np.int8).reshape(-1)), dev(xs), y, M, N, K)
     torch.cuda.synchronize()
     assert np.array_equal(host(y).reshape(M, N), want.astype(np.float32))
+
+
+@pytest.mark.parametrize("m,n", [(16, 16), (100, 200), (130, 16), (300, 257)])
+def test_mmq_integer_product_is_exact(ctx, m, n):
+    """Any int8 rows and nibbles at K = 64 under scales of 1: the exact integer
+    product, from the few-rows kernel (m <= 128) and from the tiles, whose only
+    stage here has a dead second half."""
+    print(f"mmq integer product {m}x{n}", flush=True)
+    k = 64
+    g = np.random.default_rng(m + n)
+    a = g.integers(-127, 128, (m, k))
+    b = g.integers(-8, 8, (n, k))
+    w = np.empty((n, k // 32, 18), np.uint8)
+    w[..., :2] = np.array([1.0], np.float16).view(np.uint8)
+    q = (b + 8).reshape(n, k // 32, 2, 16)
+    w[..., 2:] = q[:, :, 0] | q[:, :, 1] << 4
+    xs = np.full(m * k // 32, np.array([1.0], np.float16).view(np.uint16)[0], np.uint16)
+    y = empty(m * n, torch.float32)
+    ctx.gemm_q4_0_q8(dev(w.reshape(-1)), dev(a.astype(np.int8).reshape(-1)), dev(xs), y, m, n, k)
+    torch.cuda.synchronize()
+    assert np.array_equal(host(y).reshape(m, n), (a @ b.T).astype(np.float32))
+
+
+@pytest.mark.parametrize("m", [192, 256])
+def test_mmq_names_on_the_tiles(ctx, oracle, m):
+    """The by-name forms above 128 rows (a half-filled and a whole second row
+    tile): fp32 equal to the typed call bit for bit and within the oracle's
+    bars, f16 its sums rounded to nearest even."""
+    import sgq
+
+    print(f"mmq by name m={m}", flush=True)
+    k, n = 5376, 2048
+    rng = oracle.Rng(0x3A9 + m)
+    tw = dev(rng.random_q4_0(n * k // 32))
+    xq, xs = _quant_on_gpu(ctx, dev(oracle.through_f16(rng.f32_vec(m * k))), m, k)
+    ref, y = empty(m * n, torch.float32), empty(m * n, torch.float32)
+    y16 = torch.full((m * n + 64,), 0x7E00, dtype=torch.int16, device="cuda")
+    ctx.gemm_q4_0_q8(tw, xq, xs, ref, m, n, k)
+    B = sgq.BufferBinding.buffer
+    for name, out in (("_f32", y), ("", y16[:m * n])):
+        ctx.dispatch_blocking(ctx.load_kernel("gemm_q4_0_i8_swz_m4n1_k5376_n2048" + name),
+                              [B(0, tw), B(1, xq), B(2, xs), B(3, out)], None, [m // 64, n // 16, 1])
+    assert torch.equal(ref, y)
+    got = host(y16, np.uint16)
+    assert np.array_equal(got[:m * n], oracle.f32_to_f16_bits(host(y)))
+    assert (got[m * n:] == 0x7E00).all()
+    g = np.random.default_rng(m)
+    ms = np.concatenate([g.integers(0, m, 500), [0, 127, 128, m - 1]])
+    ns = np.concatenate([g.integers(0, n, 500), [n - 1, 0, n - 1, 0]])
+    _check_pairs(oracle, host(tw), host(xq), host(xs, np.uint16), host(y).reshape(m, n), k, ms, ns,
+                 f"by name m={m}")
+
+
+def test_mmq_rows_beyond_32_bit_offsets(ctx):
+    """K past 2^25: the last rows of a tile start beyond 4 GiB from its first,
+    where the kernel takes 64-bit offsets.  Against float64 of the same operands on a few rows; the
+    fp32 running sums of 2^17 blocks a part lose up to 2^-24 of their size each,
+    2^-24 · sqrt(2^17) = 2e-5 in the root mean square."""
+    m, n, k = 128, 2, 34_000_000
+    print(f"mmq k={k}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(25)
+    xq = torch.empty((m, k), dtype=torch.int8, device="cuda")
+    for i in range(m):
+        xq[i] = torch.randint(-127, 128, (k,), dtype=torch.int8, device="cuda", generator=g)
+    xs = (torch.rand((m, k // 32), device="cuda", generator=g) * 0.01 + 0.01).half()
+    w = torch.randint(0, 256, (n, k // 32, 18), dtype=torch.uint8, device="cuda", generator=g)
+    d = (torch.rand((n, k // 32), device="cuda", generator=g) * 0.01 + 0.01).half()
+    w[..., :2] = d.view(torch.uint8).view(n, k // 32, 2)
+    y = empty(m * n, torch.float32)
+    part = empty(8 * m * n, torch.float32)
+    ctx.gemm_q4_0_q8(w.view(-1), xq.view(-1), xs.view(torch.int16).view(-1), y, m, n, k, 8, part)
+    torch.cuda.synchronize()
+    wd = torch.cat((w[..., 2:] & 15, w[..., 2:] >> 4), -1).double().sub_(8.0).mul_(d.double()[..., None])
+    for i in (0, 1, 63, 64, 126, 127):
+        xd = xq[i].view(-1, 32).double() * xs[i].double()[:, None]
+        want = (wd * xd).sum((1, 2))
+        top = float(xd.norm() * wd[0].norm())  # the spread of such a sum
+        err = float((y.view(m, n)[i].double() - want).abs().max())
+        assert err <= 4 * 2e-5 * top, (i, err, top)
+    del xq, xs, w, wd
+    torch.cuda.empty_cache()
 
 
 def test_mmq_config2_sampled(ctx, oracle):
