@@ -396,6 +396,45 @@ def test_prefill_ipv_by_name_matches_oracle(ctx, oracle, name, q0, m):
     assert err <= 2.5e-3, (name, err)
 
 
+@pytest.mark.parametrize("tiny", ["q", "k"])
+@pytest.mark.parametrize("name", ["attn_prefill_global_flash_sp_iq", "attn_prefill_global_flash_sp_ipv"])
+def test_prefill_int8_q_with_subnormal_scales(ctx, oracle, name, tiny):
+    """int8 q or K whose f16 block scales are subnormal (values of 2^-10): the
+    scale products keep them (scores of ordinary size under a scale of 2^10, not
+    zero).  Bars as above."""
+    hd, nkv, m, q0 = 512, 4, 32, 70
+    print(f"dispatch {name} subnormal {tiny} scales", flush=True)
+    rng = oracle.Rng(0x5AB + len(name))
+    n, row = q0 + m, nkv * hd
+    small = np.float32(2.0 ** -10)
+    qs, qq = oracle.quant_q8_0(rng.f32_vec(m * NQ * hd) * (small if tiny == "q" else np.float32(1)))
+    ks, kq = oracle.quant_q8_0(rng.f32_vec(n * row) * (small if tiny == "k" else np.float32(1)))
+    assert ((qs if tiny == "q" else ks).view(np.uint16) < 0x0400).all()
+    qd, kd = oracle.dequant_q8_0(qs, qq), oracle.dequant_q8_0(ks, kq)
+    vf = rng.f32_vec(n * row)
+    out = torch.full((m * NQ * hd,), 0x7E00, dtype=torch.int16, device="cuda")
+    scale = 1024.0 / np.sqrt(hd)
+    tail = [out, _step(ctx, q0, 0, 0, q0)]
+    if name.endswith("_iq"):
+        vb = oracle.f32_to_f16_bits(vf)
+        vd, attend, bar = oracle.f16_bits_to_f32(vb), oracle.attention_head, 1.5e-3
+        binds = [dev(qq), dev(qs), dev(kq), dev(ks), dev(vb)] + tail
+    else:
+        vq, vs = np.zeros(n * row, np.int8), np.zeros(((n + 31) // 32) * row, np.uint16)
+        oracle.kv_append_v_q8(vf, n, row, 0, vq, vs)
+        vd, attend, bar = oracle.dequant_v_keyblocked(vq, vs, n, row), oracle.attention_head_ipv, 2.5e-3
+        binds = [dev(qq), dev(qs), dev(kq), dev(ks), dev(vq), dev(vs)] + tail
+    _prefill_by_name(ctx, name, binds, m, scale)
+    got = oracle.f16_bits_to_f32(host(out, np.uint16)).reshape(m, NQ, hd)
+    want = np.empty_like(got)
+    for i in range(m):
+        for h in range(NQ):
+            want[i, h] = attend(qd, kd, vd, i, h, NQ, nkv, hd, scale, 0, q0 + i)
+    top = float(np.abs(want).max())
+    assert_close(got, want, 2e-3, bar * top, name)
+    assert float(np.abs(got.astype(np.float64) - want).max()) <= bar * top
+
+
 def test_prefill_sliding_ring_equals_linear_view(ctx, oracle):
     """The two-range form (history from the pre-append ring, the chunk from
     its own pages) and the linear form over the same positions attend the
