@@ -204,3 +204,33 @@ def test_rope_vector_and_scalar_forms(ctx, oracle, head_dim, rot, n_heads):
     ctx.rope(tx, dev(cs), n_tok, n_heads, head_dim, rot)
     torch.cuda.synchronize()
     _close(host(tx), oracle.rope(x, head_dim, rot, n_heads, cs), "rope")
+
+
+@pytest.mark.parametrize("row_len", [128, 256, 512, 5376, 130])
+def test_rows_with_infinities_and_nan(ctx, oracle, row_len):
+    """Every norm form and both GeGLU forms on infinities and NaN: the
+    reference formulas' results (a row with an infinity: 0, and NaN at the
+    infinity; GeGLU of -inf: NaN)."""
+    print(f"non-finite rows of {row_len}", flush=True)
+    rows = 5
+    x = oracle.Rng(0xEA + row_len).f32_vec(rows * row_len).reshape(rows, row_len)
+    x[1, 3], x[2, 5], x[3, 7] = np.inf, -np.inf, np.nan
+    w = np.full(row_len, 2.0, np.float32)
+    y = torch.empty(rows * row_len, dtype=torch.float32, device="cuda")
+    ctx.rmsnorm(dev(x.reshape(-1)), dev(w), y, rows, row_len)
+    torch.cuda.synchronize()
+    got = host(y).reshape(rows, row_len)
+    _close(got[[0, 4]], oracle.rmsnorm(x[[0, 4]].reshape(-1), w, row_len, 1e-6, False).reshape(2, -1),
+           "finite rows")
+    for r, i in ((1, 3), (2, 5)):
+        assert np.isnan(got[r, i]) and (np.delete(got[r], i) == 0).all()
+    assert np.isnan(got[3]).all()
+
+    g = oracle.Rng(0xEB).f32_vec(rows * row_len)
+    g[:4] = np.inf, -np.inf, np.nan, 1e20
+    u = np.full(g.size, 3.0, np.float32)
+    ctx.geglu(dev(g), dev(u), y)
+    torch.cuda.synchronize()
+    got = host(y)
+    assert got[0] == np.inf and np.isnan(got[1]) and np.isnan(got[2]) and got[3] == np.float32(1e20) * 3
+    _close(got[4:], oracle.geglu(g[4:], u[4:]), "geglu")
