@@ -459,7 +459,7 @@ __global__ void splitk_reduce_kernel(const float4 *__restrict__ part, float4 *__
 // y of the tail tiles: the tail_st parts summed in part order (float4 per
 // thread, one 128×128 tile per 16 workgroups of 256 threads).
 __global__ __launch_bounds__(256) void mmq_tail_reduce_kernel(TailSplit ts, float *__restrict__ y,
-                                                              int m, int n, int mt, int nt) {
+                                                              int n, int mt, int nt) {
     const int tiles = mt * nt, lx = tiles / kXcds - ts.fx;
     const int slot = blockIdx.x / 16;  // tail tile
     const int e = (blockIdx.x % 16) * 256 + threadIdx.x;  // float4 within the tile
@@ -475,8 +475,7 @@ __global__ __launch_bounds__(256) void mmq_tail_reduce_kernel(TailSplit ts, floa
         a.z += b.z;
         a.w += b.w;
     }
-    const int row = e / (BN / 4), c4 = e % (BN / 4);
-    if (tm * BM + row >= m) return;
+    const int row = e / (BN / 4), c4 = e % (BN / 4);  // whole tiles only
     *reinterpret_cast<float4 *>(y + (size_t)(tm * BM + row) * n + tn * BN + 4 * c4) = a;
 }
 
@@ -749,7 +748,7 @@ int gemm_t(hipStream_t st, const void *w, const int8_t *xq, const uint16_t *xs, 
     if (ts.st) {
         const int tail_tiles = kXcds * (tiles / kXcds - ts.fx);
         hipLaunchKernelGGL(mmq_tail_reduce_kernel, dim3(tail_tiles * 16), dim3(256), 0, st, ts,
-                           static_cast<float *>(y), (int)m, (int)n, mt, nt);
+                           static_cast<float *>(y), (int)n, mt, nt);
         SGQ_HIP(hipGetLastError());
     }
     if (split_k > 1) {
