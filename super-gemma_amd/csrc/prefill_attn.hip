@@ -14,7 +14,7 @@
 // from the cache too.  They are dequantized to f16 as in the reference's
 // _sp_q8 variant; P is rounded to f16 for PV, as in the reference.  The
 // head_dim-256/512 kernels (below) also read the reference's other page formats
-// (PfFmt): f16 K/V (attn_prefill_px_kernel), int8 q with Q8_0 K and int8 V with
+// (PfFmt): f16 K/V (attn_prefill_pages_kernel), int8 q with Q8_0 K and int8 V with
 // key-blocked scales (attn_prefill_wide_kernel).
 //
 // Design (MFMA-bound: 4·hd flops per query-key pair against 2·hd·1 B of
@@ -724,20 +724,34 @@ __global__ __launch_bounds__(256 * HPW + 256) void attn_prefill_ws_kernel(
 //           the integer dot exact on the f16 MFMA
 //           (attn_prefill_global_flash_sp_ipv.wgsl:134-210)
 // Except for kPfQ8, q enters the MFMA as its exact f16 values and the
-// scores are scaled afterwards.  attn_prefill_px_kernel (below) serves kPfQ8H,
-// kPfF16 and all but the shortest kPfQ8.
+// scores are scaled afterwards.  prefill_px (below) does kPfQ8, kPfQ8H and kPfF16
+// but for few keys.
 enum PfFmt { kPfQ8 = 0, kPfQ8H = 1, kPfF16 = 2, kPfIQ = 3, kPfIPV = 4 };
 
+// What prefill_wide keeps in LDS (head_dim 512: 152 KB).
 template <int HD, int FMT>
-__global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
-    const void *__restrict__ qv, const uint16_t *__restrict__ q_scales, KvSource src,
-    void *__restrict__ outv, int n_tok, int q0_host, const uint32_t *__restrict__ step, int n_q,
-    int n_kv, int window, float scale, int qtiles) {
-    static_assert(FMT == kPfQ8 || FMT == kPfIQ || FMT == kPfIPV, "the others: attn_prefill_px_kernel");
+struct WideLds {
+    static constexpr int kKeys = 32, kVBuf = HD * (kKeys / 2 + 4) + HD / 16 * (kKeys / 2);  // dwords per Vᵀ buffer
+    static constexpr bool kRaw = FMT == kPfIQ || FMT == kPfIPV, kVkb = FMT == kPfIPV;
+    typedef _Float16 K[HD + 8];              // [key]
+    typedef uint32_t V[kVBuf];               // [buffer]
+    typedef float4 Ex[4][64];                // partial scores [wave][i/4][lane]
+    typedef uint16_t Ksc[HD / 32 + 4];       // int8 QK: k scales [key][block]
+    typedef float Vsk[kVkb ? HD : 1];        // kPfIPV: the tile's V scales [buffer]
+};
+
+template <int HD, int FMT>
+__device__ __forceinline__ void prefill_wide(
+    typename WideLds<HD, FMT>::K *const k_s, typename WideLds<HD, FMT>::V *const vt_s,
+    typename WideLds<HD, FMT>::Ex *const ex_s, typename WideLds<HD, FMT>::Ksc *const ksc_s,
+    typename WideLds<HD, FMT>::Vsk *const vsk_s, const void *__restrict__ qv,
+    const uint16_t *__restrict__ q_scales, const KvSource &src, void *__restrict__ outv, int n_tok,
+    int q0, int n_q, int n_kv, int window, float scale, int qtiles) {
     constexpr bool VKB = FMT == kPfIPV;  // int8 V, key-blocked scales, int8 P
-    constexpr bool QF32 = FMT == kPfQ8, KQ8 = QF32;  // K dequantized into LDS
-    constexpr bool KRAW = !QF32;                     // int8 q and K, scaled after the dots
-    constexpr bool VF16 = FMT == kPfIQ;
+    constexpr bool QF32 = FMT == kPfQ8;
+    constexpr bool KRAW = FMT == kPfIQ || VKB;           // int8 q and K, scaled after the dots
+    constexpr bool KQ8 = FMT == kPfQ8 || FMT == kPfQ8H;  // K dequantized into LDS
+    constexpr bool KF16 = FMT == kPfF16, VF16 = FMT == kPfF16 || FMT == kPfIQ;
     constexpr bool O16 = FMT != kPfQ8;
     constexpr int D = HD / 128;        // waves per query tile
     constexpr int QTW = 8 / D;         // query tiles per workgroup
@@ -746,15 +760,8 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
     constexpr int NB = HD / 32;        // 32-dim blocks per row
     constexpr int NP = KT / 2;         // key pairs per tile
     constexpr int CW = HD / 32;        // dims per staging item (8 or 16)
-    constexpr int KRow = HD + 8;       // halves
     constexpr int VS = NP + 4;         // Vᵀ row stride, dwords
-    constexpr int VBuf = HD * VS + (HD / 16) * NP;  // dwords per Vᵀ buffer
     static_assert(NP * (HD / CW) == 512, "one staging item per thread");
-    __shared__ __align__(16) _Float16 k_s[KT][KRow];
-    __shared__ __align__(16) uint32_t vt_s[2][VBuf];
-    __shared__ __align__(16) float4 ex_s[8][4][64];  // partial scores [wave][i/4][lane]
-    __shared__ __align__(16) uint16_t ksc_s[KRAW ? KT : 1][NB + 4];  // int8 QK: k scales [key][block]
-    __shared__ __align__(16) float vsk_s[VKB ? 2 : 1][VKB ? HD : 1];  // the tile's V scales
     auto vt_at = [](int row, int col) { return row * VS + (row >> 4) * NP + col; };
 
     int bx = (int)blockIdx.x, by = (int)blockIdx.y;
@@ -763,7 +770,6 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
         by = (L & 7) * per + idx % per;
         bx = idx / per;
     }
-    const int q0 = QF32 ? q0_host : (int)step[3];
     const int tile = qtiles - 1 - bx;  // heaviest (latest) query tile first
     const int qh = by, kvh = qh / (n_q / n_kv);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -791,7 +797,7 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
 #pragma unroll
                 for (int e = 0; e < 8; e++) qb[c][e] = (_Float16)(q_valid ? v[e] * qscale : 0.f);
             }
-        } else {
+        } else if constexpr (KRAW) {
             const int8_t *qr = static_cast<const int8_t *>(qv) + qoff;
 #pragma unroll
             for (int c = 0; c < 8; c++) {
@@ -804,6 +810,13 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
             const uint16_t *qs = q_scales + ((size_t)(q_valid ? my_q : 0) * n_q + qh) * NB + 4 * ds;
 #pragma unroll
             for (int b = 0; b < 4; b++) qsb[b] = q_valid ? qs[b] : 0u;
+        } else {
+            const uint16_t *qr = static_cast<const uint16_t *>(qv) + qoff;
+#pragma unroll
+            for (int c = 0; c < 8; c++) {
+                const h8 t = __builtin_bit_cast(h8, *reinterpret_cast<const uint4 *>(qr + 16 * c));
+                qb[c] = q_valid ? t : h8{};
+            }
         }
     }
 
@@ -824,7 +837,7 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
     // dims CW·chunk .. +CW-1
     const int pair = tid % NP, chunk = tid / NP;
     const int dim0 = CW * chunk, blk = dim0 >> 5;
-    constexpr int EV = VF16 ? 2 : 1;  // bytes per V element (K: 1)
+    constexpr int EK = KF16 ? 2 : 1, EV = VF16 ? 2 : 1;  // bytes per K / V element
     const char *const kq_c = sgpr_ptr(reinterpret_cast<const char *>(src.kq));
     const char *const vq_c = sgpr_ptr(reinterpret_cast<const char *>(src.vq));
     const uint16_t *const ks_c = sgpr_ptr(src.ks), *const vs_c = sgpr_ptr(src.vs);
@@ -834,7 +847,7 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
     const uint16_t *const ks_f = has_chunk ? sgpr_ptr(src.cks) : ks_c;
     const uint16_t *const vs_f = has_chunk ? sgpr_ptr(src.cvs) : vs_c;
     const int ring = src.ring;
-    typedef int kraw_t __attribute__((ext_vector_type(CW / 4)));
+    typedef int kraw_t __attribute__((ext_vector_type(CW * EK / 4)));
     typedef int vraw_t __attribute__((ext_vector_type(CW * EV / 4)));
     kraw_t rk[2];
     vraw_t rv[2];
@@ -847,9 +860,9 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
             const bool fresh = has_chunk && key >= q0;
             const int slot = fresh ? key - q0 : ring ? key % ring : key;
             const size_t row = (size_t)slot * n_kv + kvh;
-            rk[e] = gload(reinterpret_cast<const kraw_t *>((fresh ? kq_f : kq_c) + row * HD + dim0));
+            rk[e] = gload(reinterpret_cast<const kraw_t *>((fresh ? kq_f : kq_c) + (row * HD + dim0) * EK));
             rv[e] = gload(reinterpret_cast<const vraw_t *>((fresh ? vq_f : vq_c) + (row * HD + dim0) * EV));
-            rsk[e] = gload((fresh ? ks_f : ks_c) + row * NB + blk);
+            if constexpr (!KF16) rsk[e] = gload((fresh ? ks_f : ks_c) + row * NB + blk);
             if constexpr (!VF16 && !VKB) rsv[e] = gload((fresh ? vs_f : vs_c) + row * NB + blk);
         }
         if constexpr (VKB)
@@ -868,22 +881,30 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
             const bool live = kl + kk <= k_hi;
             h8 kt[CW / 8];
             _Float16 vv[CW];
-            const _Float16 sk = KQ8 && live ? __builtin_bit_cast(_Float16, rsk[e]) : (_Float16)1.f;
-            const h2 dk = {sk, sk};
+            if constexpr (KF16) {
 #pragma unroll
-            for (int w = 0; w < CW / 4; w++) {
-                h2 k01 = i8_pair_f16((uint32_t)rk[e][w], 0x04010400u);
-                h2 k23 = i8_pair_f16((uint32_t)rk[e][w], 0x04030402u);
-                if constexpr (KQ8) k01 *= dk, k23 *= dk;
-                kt[w / 2][4 * (w & 1)] = k01[0], kt[w / 2][4 * (w & 1) + 1] = k01[1];
-                kt[w / 2][4 * (w & 1) + 2] = k23[0], kt[w / 2][4 * (w & 1) + 3] = k23[1];
+                for (int h = 0; h < CW / 8; h++) {
+                    const int4 t = {rk[e][4 * h], rk[e][4 * h + 1], rk[e][4 * h + 2], rk[e][4 * h + 3]};
+                    kt[h] = live ? __builtin_bit_cast(h8, t) : h8{};
+                }
+            } else {
+                const _Float16 sk = KQ8 && live ? __builtin_bit_cast(_Float16, rsk[e]) : (_Float16)1.f;
+                const h2 dk = {sk, sk};
+#pragma unroll
+                for (int w = 0; w < CW / 4; w++) {
+                    h2 k01 = i8_pair_f16((uint32_t)rk[e][w], 0x04010400u);
+                    h2 k23 = i8_pair_f16((uint32_t)rk[e][w], 0x04030402u);
+                    if constexpr (KQ8) k01 *= dk, k23 *= dk;
+                    kt[w / 2][4 * (w & 1)] = k01[0], kt[w / 2][4 * (w & 1) + 1] = k01[1];
+                    kt[w / 2][4 * (w & 1) + 2] = k23[0], kt[w / 2][4 * (w & 1) + 3] = k23[1];
+                }
+                if (!live)
+#pragma unroll
+                    for (int h = 0; h < CW / 8; h++) kt[h] = h8{};
+                if constexpr (KRAW)
+                    if (dim0 % 32 == 0)
+                        ksc_s[kk][blk] = live ? rsk[e] : (uint16_t)0;
             }
-            if (!live)
-#pragma unroll
-                for (int h = 0; h < CW / 8; h++) kt[h] = h8{};
-            if constexpr (KRAW)
-                if (dim0 % 32 == 0)
-                    ksc_s[kk][blk] = live ? rsk[e] : (uint16_t)0;
             if constexpr (VF16) {
 #pragma unroll
                 for (int w = 0; w < CW / 2; w++) {
@@ -984,7 +1005,7 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
             }
             s[4 * j] = t.x, s[4 * j + 1] = t.y, s[4 * j + 2] = t.z, s[4 * j + 3] = t.w;
         }
-        if constexpr (KRAW)
+        if constexpr (!QF32)
 #pragma unroll
             for (int i = 0; i < 16; i++) s[i] *= qscale;
         const uint32_t *vt = vt_s[buf];
@@ -1101,6 +1122,22 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
         }
 }
 
+template <int HD, int FMT>
+__global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
+    const void *__restrict__ qv, const uint16_t *__restrict__ q_scales, KvSource src,
+    void *__restrict__ outv, int n_tok, int q0_host, const uint32_t *__restrict__ step, int n_q,
+    int n_kv, int window, float scale, int qtiles) {
+    static_assert(FMT == kPfQ8 || FMT == kPfIQ || FMT == kPfIPV, "the others: attn_prefill_pages_kernel");
+    typedef WideLds<HD, FMT> L;
+    __shared__ __align__(16) typename L::K k_s[L::kKeys];
+    __shared__ __align__(16) typename L::V vt_s[2];
+    __shared__ __align__(16) typename L::Ex ex_s[8];
+    __shared__ __align__(16) typename L::Ksc ksc_s[L::kRaw ? L::kKeys : 1];
+    __shared__ __align__(16) typename L::Vsk vsk_s[L::kVkb ? 2 : 1];
+    prefill_wide<HD, FMT>(k_s, vt_s, ex_s, ksc_s, vsk_s, qv, q_scales, src, outv, n_tok,
+                          FMT == kPfQ8 ? q0_host : (int)step[3], n_q, n_kv, window, scale, qtiles);
+}
+
 // The larger of a lane's value and that of the lane 32 (16) away, without the
 // LDS trip of a shuffle.
 __device__ __forceinline__ float max_x32(float v) {
@@ -1115,7 +1152,7 @@ __device__ __forceinline__ float max_x16(float v) {
     return fmaxf(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
 }
 
-// Prefill attention at head_dim 256 / 512 without repeated scores: one query
+// prefill_px: prefill attention at head_dim 256 / 512 without repeated scores.  One query
 // head per workgroup of 8 waves, D = head_dim/128 waves per tile of 32 queries.
 // A tile's scores are cut between its D waves by (key, query), over all dims,
 // so that no score is computed, masked or exponentiated twice:
@@ -1127,7 +1164,7 @@ __device__ __forceinline__ float max_x16(float v) {
 // whole P as the B operand of Oᵀ = Vᵀ·Pᵀ for its own 128 dims.  At head_dim 256
 // a wave has 32 keys of a query, rounds them to f16 and writes their fp32 sum
 // beside them; at 512 P goes through LDS in fp32, and the readers sum and round.
-// The numerics are attn_prefill_wide_kernel's, bit for bit: scores, fp32
+// The numerics are prefill_wide's, bit for bit: scores, fp32
 // denominators and outputs are summed in its order, under one reference maximum
 // per query and 32 keys, which moves when the maximum has passed it by 2^8.  P is
 // written for the reference as it stands.  A wave that finds that a reference has
@@ -1135,7 +1172,7 @@ __device__ __forceinline__ float max_x16(float v) {
 // takes one more barrier to agree on the references and write P again.
 // Per tile: scores, P out → barrier → K(t+1) and V(t+1) staged from registers
 // (V double-buffered), quants of t+2 issued, PV(t) → barrier.
-// Against attn_prefill_wide_kernel, whose D waves each compute partial scores
+// Against prefill_wide, whose D waves each compute partial scores
 // over 128 dims, exchange them as fp32 and repeat the softmax (us, wide -> here;
 // kv heads 16 / 4): head_dim 256, Q8_0, 1024 window, 4096 queries 401 -> 311,
 // 1111 queries from 2003 195 -> 156; f16 ring, 512 queries from 1777 84 -> 72;
@@ -1149,33 +1186,41 @@ __device__ __forceinline__ float max_x16(float v) {
 // kernel's scores with only the softmax cut (2000 queries of 512: 429).  Int8 q
 // stays with the wide kernel: here its block scales spill (322 -> 1020 for 1024
 // queries from 1024).
+template <int HD>
+struct PxLds {
+    static constexpr bool S32 = HD == 256;
+    static constexpr int kQueries = 32 * (8 / (HD / 128)), kKeys = S32 ? 64 : 32;
+    static constexpr int KRowB = (HD + 8) * 2;      // bytes per K row (f16)
+    static constexpr int VS = kKeys / 2 + 4;        // Vᵀ row, dwords (16-byte reads, 4 banks apart)
+    static constexpr int VPad = S32 ? 0 : 16;       // dwords per 16 rows: the staging writes of a wave
+    static constexpr int VBuf = HD * VS + (HD / 16) * VPad;
+    static constexpr int PRow = kKeys + 8;          // P row (halves, S32): [query][key, in operand order]
+    static constexpr int kKBytes = kKeys * KRowB, kVBytes = 2 * VBuf * 4;
+    static constexpr int kPBytes = S32 ? kQueries * PRow * 2 : kQueries * 32 * 4;
+    static constexpr int kMBytes = 4 * kQueries * 4;  // [key part][query]: maxima, then (S32) sums of P
+    static constexpr int kBytes = kKBytes + kVBytes + kPBytes + kMBytes;
+};
+
+// moved[2]: a reference moves in this tile / the next.
 template <int HD, int FMT>
-__global__ __launch_bounds__(512, 2) void attn_prefill_px_kernel(
-    const void *__restrict__ qv, const uint16_t *__restrict__ q_scales, KvSource src,
-    void *__restrict__ outv, int n_tok, int q0_host, const uint32_t *__restrict__ step, int n_q,
-    int n_kv, int window, float scale, int qtiles) {
+__device__ __forceinline__ void prefill_px(uint8_t *const lds, uint32_t *const moved,
+                                           const void *__restrict__ qv, const KvSource &src,
+                                           void *__restrict__ outv, int n_tok, int q0, int n_q,
+                                           int n_kv, int window, float scale, int qtiles) {
+    typedef PxLds<HD> L;
     constexpr bool QF32 = FMT == kPfQ8, F16 = FMT == kPfF16, O16 = FMT != kPfQ8;
     static_assert(QF32 || F16 || FMT == kPfQ8H, "Q8_0 or f16 pages, fp32 or f16 q");
     constexpr bool S32 = HD == 256;           // scores as a 32×32 tile (else 16×16)
     constexpr int D = HD / 128;               // waves per query tile
-    constexpr int QW = 32 * (8 / D);          // queries per workgroup
-    constexpr int KT = S32 ? 64 : 32, G = KT / 32;  // keys per tile, 32 to a reference
+    constexpr int QW = L::kQueries;           // queries per workgroup
+    constexpr int KT = L::kKeys, G = KT / 32;  // keys per tile, 32 to a reference
     constexpr int NB = HD / 32, NP = KT / 2, CW = 16;
     static_assert(NP * (HD / CW) == 512, "one staging item per thread");
-    constexpr int KRowB = (HD + 8) * 2;       // bytes per K row (f16) in LDS
-    constexpr int VS = NP + 4;                // Vᵀ row, dwords (16-byte reads, 4 banks apart)
-    constexpr int VPad = S32 ? 0 : 16;        // dwords per 16 rows: the staging writes of a wave
-    constexpr int VBuf = HD * VS + (HD / 16) * VPad;
-    constexpr int PRow = KT + 8;              // P row (halves, S32): [query][key, in operand order]
-    constexpr int kPBytes = S32 ? QW * PRow * 2 : QW * 32 * 4;
-    constexpr int kKBytes = KT * KRowB, kVBytes = 2 * VBuf * 4;
-    constexpr int kMBytes = 4 * QW * 4;       // [key part][query]: maxima, then (S32) sums of P
-    __shared__ __align__(16) uint8_t lds[kKBytes + kVBytes + kPBytes + kMBytes];
-    __shared__ uint32_t moved[2];             // a reference moves in this tile / the next
+    constexpr int KRowB = L::KRowB, VS = L::VS, VPad = L::VPad, VBuf = L::VBuf, PRow = L::PRow;
     uint8_t *const k_lds = lds;
-    uint32_t *const v_lds = reinterpret_cast<uint32_t *>(lds + kKBytes);
-    uint16_t *const p_lds = reinterpret_cast<uint16_t *>(lds + kKBytes + kVBytes);
-    float *const m_lds = reinterpret_cast<float *>(lds + kKBytes + kVBytes + kPBytes);
+    uint32_t *const v_lds = reinterpret_cast<uint32_t *>(lds + L::kKBytes);
+    uint16_t *const p_lds = reinterpret_cast<uint16_t *>(lds + L::kKBytes + L::kVBytes);
+    float *const m_lds = reinterpret_cast<float *>(lds + L::kKBytes + L::kVBytes + L::kPBytes);
     float *const l_lds = m_lds + 2 * QW;
     auto vt_at = [](int row, int col) { return row * VS + (row >> 4) * VPad + col; };
 
@@ -1185,7 +1230,6 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_px_kernel(
         by = (L & 7) * per + idx % per;
         bx = idx / per;
     }
-    const int q0 = QF32 ? q0_host : (int)step[3];
     const int tile = qtiles - 1 - bx;  // heaviest (latest) query tile first
     const int qh = by, kvh = qh / (n_q / n_kv);
     const int tid = threadIdx.x, lane = tid & 63;
@@ -1534,6 +1578,42 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_px_kernel(
         }
 }
 
+template <int HD>
+__global__ __launch_bounds__(512, 2) void attn_prefill_px_kernel(
+    const void *__restrict__ qv, const uint16_t *, KvSource src, void *__restrict__ outv, int n_tok,
+    int q0, const uint32_t *, int n_q, int n_kv, int window, float scale, int qtiles) {
+    __shared__ __align__(16) uint8_t lds[PxLds<HD>::kBytes];
+    __shared__ uint32_t moved[2];
+    prefill_px<HD, kPfQ8>(lds, moved, qv, src, outv, n_tok, q0, n_q, n_kv, window, scale, qtiles);
+}
+
+// The forms dispatched by name.  Their position, and with it the number of keys,
+// is known on the device only, so the choice between the two ways is made here.
+// us, prefill_wide / prefill_px as kernels of their own / here: head_dim 256, 16 /
+// 32 / 48 / 64 keys 6.5 / 7.8 / 6.7, 7.2 / 8.7 / 7.5, 10.1 / 10.0 / 10.3, 10.5 /
+// 11.0 / 10.9; 512, as many queries as keys, 64 / 128 / 160 / 192 15.4 / 16.4 / 15.6, 20.4 / 21.4 / 21.0,
+// 20.9 / 21.8 / 21.4, 26.4 / 26.8 / 26.6 (f16; Q8_0 the same within 0.3); 16
+// queries, 48 / 80 keys 11.0 / 11.0, 13.7 / 13.1.  LDS is the larger of both: one
+// workgroup per CU either way.
+template <int HD, int FMT>
+__global__ __launch_bounds__(512, 2) void attn_prefill_pages_kernel(
+    const void *__restrict__ qv, const uint16_t *, KvSource src, void *__restrict__ outv, int n_tok,
+    int, const uint32_t *__restrict__ step, int n_q, int n_kv, int window, float scale, int qtiles) {
+    typedef WideLds<HD, FMT> L;
+    constexpr int kKB = L::kKeys * (int)sizeof(typename L::K), kVB = 2 * (int)sizeof(typename L::V);
+    constexpr int kWide = kKB + kVB + 8 * (int)sizeof(typename L::Ex);
+    __shared__ __align__(16) uint8_t lds[kWide > PxLds<HD>::kBytes ? kWide : PxLds<HD>::kBytes];
+    __shared__ uint32_t moved[2];
+    const int q0 = (int)step[3];
+    if (q0 + n_tok <= (HD == 256 ? 64 : n_tok > 32 ? 160 : 32))
+        prefill_wide<HD, FMT>(reinterpret_cast<typename L::K *>(lds),
+                              reinterpret_cast<typename L::V *>(lds + kKB),
+                              reinterpret_cast<typename L::Ex *>(lds + kKB + kVB), nullptr, nullptr,
+                              qv, nullptr, src, outv, n_tok, q0, n_q, n_kv, window, scale, qtiles);
+    else
+        prefill_px<HD, FMT>(lds, moved, qv, src, outv, n_tok, q0, n_q, n_kv, window, scale, qtiles);
+}
+
 }  // namespace
 
 int launch_attn_prefill_ipv(hipStream_t st, const float *q, const int8_t *kq, const uint16_t *ks,
@@ -1594,15 +1674,15 @@ int launch_attn_prefill_q8(hipStream_t st, const float *q, const int8_t *kq, con
         // 100 / 200 / 320 keys 18.4 / 26.4 / 33.4 against 18.3 / 24.2 / 29.7.
         const int n_keys = q0 + n_tok;
         const bool few_keys = n_keys <= (head_dim == 256 ? 32 : n_tok > 32 ? 512 : 96);
-#define SGQ_PF_Q8(KERNEL, HD)                                                                    \
-    hipLaunchKernelGGL((KERNEL<HD, kPfQ8>), grid, dim3(512), 0, st, q, no_qs, src, out, n_tok, q0, \
+#define SGQ_PF_Q8(...)                                                                           \
+    hipLaunchKernelGGL((__VA_ARGS__), grid, dim3(512), 0, st, q, no_qs, src, out, n_tok, q0, \
                        no_step, n_q, n_kv, window, scale, (int)grid.x)
         if (head_dim == 256) {
-            if (few_keys) SGQ_PF_Q8(attn_prefill_wide_kernel, 256);
-            else SGQ_PF_Q8(attn_prefill_px_kernel, 256);
+            if (few_keys) SGQ_PF_Q8(attn_prefill_wide_kernel<256, kPfQ8>);
+            else SGQ_PF_Q8(attn_prefill_px_kernel<256>);
         } else {
-            if (few_keys) SGQ_PF_Q8(attn_prefill_wide_kernel, 512);
-            else SGQ_PF_Q8(attn_prefill_px_kernel, 512);
+            if (few_keys) SGQ_PF_Q8(attn_prefill_wide_kernel<512, kPfQ8>);
+            else SGQ_PF_Q8(attn_prefill_px_kernel<512>);
         }
 #undef SGQ_PF_Q8
         SGQ_HIP(hipGetLastError());
@@ -1653,13 +1733,13 @@ int launch_attn_prefill_pages(hipStream_t st, int fmt, const void *q, const uint
     hipLaunchKernelGGL((KERNEL<HD, F>), grid, dim3(512), 0, st, q, q_scales, src, out, n_tok, 0,     \
                        step, n_q, n_kv, window, scale, qt)
     if (head_dim == 256) {
-        if (fmt == kPfQ8H) SGQ_PF_PAGES(attn_prefill_px_kernel, 256, kPfQ8H);
-        else if (fmt == kPfF16) SGQ_PF_PAGES(attn_prefill_px_kernel, 256, kPfF16);
+        if (fmt == kPfQ8H) SGQ_PF_PAGES(attn_prefill_pages_kernel, 256, kPfQ8H);
+        else if (fmt == kPfF16) SGQ_PF_PAGES(attn_prefill_pages_kernel, 256, kPfF16);
         else if (fmt == kPfIQ) SGQ_PF_PAGES(attn_prefill_wide_kernel, 256, kPfIQ);
         else SGQ_PF_PAGES(attn_prefill_wide_kernel, 256, kPfIPV);
     } else {
-        if (fmt == kPfQ8H) SGQ_PF_PAGES(attn_prefill_px_kernel, 512, kPfQ8H);
-        else if (fmt == kPfF16) SGQ_PF_PAGES(attn_prefill_px_kernel, 512, kPfF16);
+        if (fmt == kPfQ8H) SGQ_PF_PAGES(attn_prefill_pages_kernel, 512, kPfQ8H);
+        else if (fmt == kPfF16) SGQ_PF_PAGES(attn_prefill_pages_kernel, 512, kPfF16);
         else if (fmt == kPfIQ) SGQ_PF_PAGES(attn_prefill_wide_kernel, 512, kPfIQ);
         else SGQ_PF_PAGES(attn_prefill_wide_kernel, 512, kPfIPV);
     }

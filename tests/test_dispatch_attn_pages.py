@@ -435,6 +435,51 @@ def test_prefill_int8_q_with_subnormal_scales(ctx, oracle, name, tiny):
     assert float(np.abs(got.astype(np.float64) - want).max()) <= bar * top
 
 
+@pytest.mark.parametrize("name,q0,short,long_", [
+    ("attn_prefill_sliding_ring", 0, 48, 80), ("attn_prefill_sliding_ring", 30, 32, 160),
+    ("attn_prefill_sliding", 0, 63, 66), ("attn_prefill_global_flash_sp", 0, 16, 48),
+    ("attn_prefill_global_flash_sp", 0, 160, 176), ("attn_prefill_global_flash_sp", 90, 64, 96),
+    ("attn_prefill_global_flash_sp_q8", 0, 32, 192), ("attn_prefill_global_flash_sp_q8", 16, 16, 160)])
+def test_prefill_pages_rows_do_not_depend_on_the_chunk(ctx, oracle, name, q0, short, long_):
+    """The kernel behind these names takes one way with few keys (64 at head_dim
+    256; at 512 160, or 32 for at most 32 queries) and another with more: the rows
+    that a short and a long chunk share have the same bits, also where a reference
+    maximum moves (later keys four times as large).  The short chunk is within the
+    oracle's bars."""
+    hd, nkv, window, _ = PREFILL[name]
+    print(f"dispatch {name} q0={q0} {short}/{long_}", flush=True)
+    rng = oracle.Rng(0xC41 + q0 + long_ + hd)
+    row = nkv * hd
+    kf, vf = (rng.f32_vec((q0 + long_) * row) for _ in range(2))
+    kf.reshape(-1, row)[(q0 + short) // 3:] *= np.float32(4.0)
+    q16 = oracle.f32_to_f16_bits(rng.f32_vec(long_ * NQ * hd))
+    scale, got = 2.0 / np.sqrt(hd), []
+    for m in (short, long_):
+        n = (q0 + m) * row
+        if name.endswith("_q8"):
+            (ks, kq), (vs, vq) = oracle.quant_q8_0(kf[:n]), oracle.quant_q8_0(vf[:n])
+            kd, vd = oracle.dequant_q8_0_f16(ks, kq), oracle.dequant_q8_0_f16(vs, vq)
+            pages = [dev(kq), dev(ks), dev(vq), dev(vs)]
+        else:
+            kb, vb = oracle.f32_to_f16_bits(kf[:n]), oracle.f32_to_f16_bits(vf[:n])
+            kd, vd = oracle.f16_bits_to_f32(kb), oracle.f16_bits_to_f32(vb)
+            pages = [dev(kb), dev(vb)]
+            if name.endswith("_ring"):
+                old = [np.full(RING * row, 0x7E00, np.uint16) for _ in range(2)]
+                for o, b in zip(old, (kb, vb)):
+                    o[:q0 * row] = b[:q0 * row]
+                pages = [dev(o) for o in old] + [dev(kb[q0 * row:]), dev(vb[q0 * row:])]
+        out = torch.full((m * NQ * hd,), 0x7E00, dtype=torch.int16, device="cuda")
+        _prefill_by_name(ctx, name, [dev(q16[:m * NQ * hd])] + pages + [out, _step(ctx, q0, 0, 0, q0)],
+                         m, scale)
+        got.append(host(out, np.uint16).reshape(m, NQ, hd)[:short])
+        if m == short:
+            _prefill_check(oracle.f16_bits_to_f32(got[0]).reshape(m, NQ, hd),
+                           oracle.attention(oracle.f16_bits_to_f32(q16[:m * NQ * hd]), kd, vd, m, q0, NQ,
+                                            nkv, hd, window, scale), f"{name} few keys")
+    assert np.array_equal(got[0], got[1])
+
+
 def test_prefill_sliding_ring_equals_linear_view(ctx, oracle):
     """The two-range form (history from the pre-append ring, the chunk from
     its own pages) and the linear form over the same positions attend the
