@@ -664,11 +664,16 @@ void skinny_launch(hipStream_t st, const void *w, const int8_t *xq, const uint16
 // time grows with n by 1.0 / 1.8 / 3.6 us per 1000 columns (M <= 32 / 64 /
 // 128, K = 5376) where the tiles' stays until their round of 65536 columns is
 // full, hence the limits on n; above 64 rows a caller's split over K is the
-// faster of the two.
-bool skinny(uint32_t m, uint32_t n, uint32_t split_k) {
+// faster of the two.  Above 96 rows 16384 columns are one round of the few-rows
+// workgroups, and the second costs more than the tiles' (128 rows, N = 21504,
+// tiles / few rows: K = 512 12.3 / 16.4, 21504 312 / 375; N = 16384 12.2 / 11.6,
+// 312 / 175).  A K of a few blocks leaves most of the waves that cut it idle (K =
+// 64, N = 21504: 65 rows 6.7 / 9.4, 128 rows 7.5 / 13.0; from K = 512 on it pays).
+bool skinny(uint32_t m, uint32_t n, uint32_t k, uint32_t split_k) {
     if (m <= 32) return true;
+    if (k < 256 && n > 8192) return false;
     if (m <= 64) return n <= 43008;
-    return m <= 128 && n <= 21504 && split_k == 1;
+    return m <= 128 && n <= (m <= 96 ? 21504 : 16384) && split_k == 1;
 }
 
 template <bool HOUT>
@@ -684,7 +689,7 @@ int gemm_t(hipStream_t st, const void *w, const int8_t *xq, const uint16_t *xs, 
     SGQ_CHECK(((uintptr_t)w & 3) == 0, "gemm_q4_0_q8: weights must be 4-byte aligned");
     SGQ_CHECK((uint64_t)m * n < (1ull << 31) * 4, "gemm_q4_0_q8: output too large");
     SGQ_CHECK(split_k == 1 || (m * (uint64_t)n) % 4 == 0, "gemm_q4_0_q8: m*n must be a multiple of 4 for split-K");
-    if (k < kWideK && skinny(m, n, split_k)) {
+    if (k < kWideK && skinny(m, n, k, split_k)) {
         // W: 8 waves cut a column tile's K finer (N = 5376, K = 21504, M = 37:
         // 43 against 69 us); with two tiles or more per CU, 4 leave smaller
         // workgroups to even out over the CUs (N = 21504, M = 37: 35 against 45)

@@ -61,6 +61,7 @@ def test_mmq_small_full_check(ctx, oracle, m, k, n):
     (128, 320, 131, 1), (65, 1088, 132, 4), (300, 2112, 260, 8),
     (16, 128, 31, 1), (31, 2112, 96, 8), (32, 64, 33, 1), (64, 1088, 65, 2), (96, 192, 64, 1),
     (97, 576, 37, 1), (2, 192, 16390, 1), (40, 128, 16385, 1), (100, 128, 16390, 1),
+    (40, 256, 16385, 1), (100, 256, 16384, 1), (100, 256, 16385, 1), (96, 256, 21504, 1), (65, 192, 8196, 1),
     (129, 64, 127, 1), (132, 64, 130, 8), (132, 192, 130, 2), (132, 192, 130, 4)])
 def test_mmq_tile_and_k_edges(ctx, oracle, m, k, n, split):
     """Rows and columns around the tile edges with a K that ends in two
@@ -68,8 +69,9 @@ def test_mmq_tile_and_k_edges(ctx, oracle, m, k, n, split):
     into more parts than K has stages and with a last part of two blocks:
     every element against the oracle, the operands at the very end of their
     buffers and the output's surroundings untouched.  Up to 64 rows (128
-    unsplit) the few-rows kernel answers: its row tiles' edges, K ranges
-    shorter than its waves, and both workgroup sizes."""
+    unsplit) the few-rows kernel answers, within limits on N and K: its row
+    tiles' edges, K ranges shorter than its waves, both workgroup sizes, and
+    either side of those limits."""
     print(f"mmq edges m={m} k={k} n={n} split={split}", flush=True)
     rng = oracle.Rng(0xED6E + m + k + n)
     w = rng.random_q4_0(n * k // 32)
