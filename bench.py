@@ -349,7 +349,7 @@ class AttnPrefillPages:
         import struct
         import sgq
 
-        self.kernel = ("attn_prefill_pages_kernel" if kind == "sliding_ring"
+        self.kernel = ("attn_prefill_px_kernel" if kind == "sliding_ring"
                        else "attn_prefill_wide_kernel")
         self.ctx, self.kind, self.n_tok = ctx, kind, n_tok
         n_q = 32

@@ -14,7 +14,7 @@
 // from the cache too.  They are dequantized to f16 as in the reference's
 // _sp_q8 variant; P is rounded to f16 for PV, as in the reference.  The
 // head_dim-256/512 kernels (below) also read the reference's other page formats
-// (PfFmt): f16 K/V (attn_prefill_pages_kernel), int8 q with Q8_0 K and int8 V with
+// (PfFmt): f16 K/V (attn_prefill_px_kernel), int8 q with Q8_0 K and int8 V with
 // key-blocked scales (attn_prefill_wide_kernel).
 //
 // Design (MFMA-bound: 4·hd flops per query-key pair against 2·hd·1 B of
@@ -724,9 +724,14 @@ __global__ __launch_bounds__(256 * HPW + 256) void attn_prefill_ws_kernel(
 //           the integer dot exact on the f16 MFMA
 //           (attn_prefill_global_flash_sp_ipv.wgsl:134-210)
 // Except for kPfQ8, q enters the MFMA as its exact f16 values and the
-// scores are scaled afterwards.  prefill_px (below) does kPfQ8, kPfQ8H and kPfF16
-// but for few keys.
+// scores are scaled afterwards.  attn_prefill_px_kernel (below) does kPfQ8,
+// kPfQ8H and kPfF16 but for few keys.
 enum PfFmt { kPfQ8 = 0, kPfQ8H = 1, kPfF16 = 2, kPfIQ = 3, kPfIPV = 4 };
+
+// Query loads as native vectors: of HIP's float4, a struct, the compiler put single
+// words into branches of their own where a lane may have no query (head_dim 512,
+// 64 keys 18.1 -> 19.2 us).
+typedef float f4_q __attribute__((ext_vector_type(4)));
 
 // What prefill_wide keeps in LDS (head_dim 512: 152 KB).
 template <int HD, int FMT>
@@ -791,9 +796,9 @@ __device__ __forceinline__ void prefill_wide(
             const float *qr = static_cast<const float *>(qv) + qoff;
 #pragma unroll
             for (int c = 0; c < 8; c++) {
-                const float4 a = *reinterpret_cast<const float4 *>(qr + 16 * c);
-                const float4 b = *reinterpret_cast<const float4 *>(qr + 16 * c + 4);
-                const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+                const f4_q a = *reinterpret_cast<const f4_q *>(qr + 16 * c);
+                const f4_q b = *reinterpret_cast<const f4_q *>(qr + 16 * c + 4);
+                const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
 #pragma unroll
                 for (int e = 0; e < 8; e++) qb[c][e] = (_Float16)(q_valid ? v[e] * qscale : 0.f);
             }
@@ -814,7 +819,7 @@ __device__ __forceinline__ void prefill_wide(
             const uint16_t *qr = static_cast<const uint16_t *>(qv) + qoff;
 #pragma unroll
             for (int c = 0; c < 8; c++) {
-                const h8 t = __builtin_bit_cast(h8, *reinterpret_cast<const uint4 *>(qr + 16 * c));
+                const h8 t = *reinterpret_cast<const h8 *>(qr + 16 * c);
                 qb[c] = q_valid ? t : h8{};
             }
         }
@@ -1127,7 +1132,7 @@ __global__ __launch_bounds__(512) void attn_prefill_wide_kernel(
     const void *__restrict__ qv, const uint16_t *__restrict__ q_scales, KvSource src,
     void *__restrict__ outv, int n_tok, int q0_host, const uint32_t *__restrict__ step, int n_q,
     int n_kv, int window, float scale, int qtiles) {
-    static_assert(FMT == kPfQ8 || FMT == kPfIQ || FMT == kPfIPV, "the others: attn_prefill_pages_kernel");
+    static_assert(FMT == kPfQ8 || FMT == kPfIQ || FMT == kPfIPV, "the others: attn_prefill_px_kernel");
     typedef WideLds<HD, FMT> L;
     __shared__ __align__(16) typename L::K k_s[L::kKeys];
     __shared__ __align__(16) typename L::V vt_s[2];
@@ -1152,7 +1157,7 @@ __device__ __forceinline__ float max_x16(float v) {
     return fmaxf(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
 }
 
-// prefill_px: prefill attention at head_dim 256 / 512 without repeated scores.  One query
+// Prefill attention at head_dim 256 / 512 without repeated scores: one query
 // head per workgroup of 8 waves, D = head_dim/128 waves per tile of 32 queries.
 // A tile's scores are cut between its D waves by (key, query), over all dims,
 // so that no score is computed, masked or exponentiated twice:
@@ -1186,43 +1191,58 @@ __device__ __forceinline__ float max_x16(float v) {
 // kernel's scores with only the softmax cut (2000 queries of 512: 429).  Int8 q
 // stays with the wide kernel: here its block scales spill (322 -> 1020 for 1024
 // queries from 1024).
-template <int HD>
-struct PxLds {
-    static constexpr bool S32 = HD == 256;
-    static constexpr int kQueries = 32 * (8 / (HD / 128)), kKeys = S32 ? 64 : 32;
-    static constexpr int KRowB = (HD + 8) * 2;      // bytes per K row (f16)
-    static constexpr int VS = kKeys / 2 + 4;        // Vᵀ row, dwords (16-byte reads, 4 banks apart)
-    static constexpr int VPad = S32 ? 0 : 16;       // dwords per 16 rows: the staging writes of a wave
-    static constexpr int VBuf = HD * VS + (HD / 16) * VPad;
-    static constexpr int PRow = kKeys + 8;          // P row (halves, S32): [query][key, in operand order]
-    static constexpr int kKBytes = kKeys * KRowB, kVBytes = 2 * VBuf * 4;
-    static constexpr int kPBytes = S32 ? kQueries * PRow * 2 : kQueries * 32 * 4;
-    static constexpr int kMBytes = 4 * kQueries * 4;  // [key part][query]: maxima, then (S32) sums of P
-    static constexpr int kBytes = kKBytes + kVBytes + kPBytes + kMBytes;
-};
-
-// moved[2]: a reference moves in this tile / the next.
+//
+// The forms dispatched by name get their position from the device, and with it the
+// number of keys, so this kernel decides for them whether there are so few that
+// prefill_wide's way is shorter.  us, prefill_wide / this without it / with it:
+// head_dim 256, 16 / 32 / 48 / 64 keys 6.5 / 7.8 / 6.7, 7.2 / 8.7 / 7.5, 10.1 / 10.1 /
+// 10.4, 10.5 / 11.0 / 10.9, 80 and 96 13.3 / 15.2, 13.8 / 15.9; 512, as many queries as keys, 64 / 128 / 160 / 192 15.4 /
+// 16.4 / 15.6, 20.4 / 21.4 / 21.0, 20.9 / 21.8 / 21.4, 26.4 / 26.8 / 26.6 (f16; Q8_0
+// the same within 0.3); 16 queries, 48 / 80 keys 11.0 / 11.0, 13.7 / 13.1.
 template <int HD, int FMT>
-__device__ __forceinline__ void prefill_px(uint8_t *const lds, uint32_t *const moved,
-                                           const void *__restrict__ qv, const KvSource &src,
-                                           void *__restrict__ outv, int n_tok, int q0, int n_q,
-                                           int n_kv, int window, float scale, int qtiles) {
-    typedef PxLds<HD> L;
+__global__ __launch_bounds__(512, 2) void attn_prefill_px_kernel(
+    const void *__restrict__ qv, const uint16_t *__restrict__ q_scales, KvSource src,
+    void *__restrict__ outv, int n_tok, int q0_host, const uint32_t *__restrict__ step, int n_q,
+    int n_kv, int window, float scale, int qtiles) {
     constexpr bool QF32 = FMT == kPfQ8, F16 = FMT == kPfF16, O16 = FMT != kPfQ8;
     static_assert(QF32 || F16 || FMT == kPfQ8H, "Q8_0 or f16 pages, fp32 or f16 q");
     constexpr bool S32 = HD == 256;           // scores as a 32×32 tile (else 16×16)
     constexpr int D = HD / 128;               // waves per query tile
-    constexpr int QW = L::kQueries;           // queries per workgroup
-    constexpr int KT = L::kKeys, G = KT / 32;  // keys per tile, 32 to a reference
+    constexpr int QW = 32 * (8 / D);          // queries per workgroup
+    constexpr int KT = S32 ? 64 : 32, G = KT / 32;  // keys per tile, 32 to a reference
     constexpr int NB = HD / 32, NP = KT / 2, CW = 16;
     static_assert(NP * (HD / CW) == 512, "one staging item per thread");
-    constexpr int KRowB = L::KRowB, VS = L::VS, VPad = L::VPad, VBuf = L::VBuf, PRow = L::PRow;
+    constexpr int KRowB = (HD + 8) * 2;       // bytes per K row (f16) in LDS
+    constexpr int VS = NP + 4;                // Vᵀ row, dwords (16-byte reads, 4 banks apart)
+    constexpr int VPad = S32 ? 0 : 16;        // dwords per 16 rows: the staging writes of a wave
+    constexpr int VBuf = HD * VS + (HD / 16) * VPad;
+    constexpr int PRow = KT + 8;              // P row (halves, S32): [query][key, in operand order]
+    constexpr int kPBytes = S32 ? QW * PRow * 2 : QW * 32 * 4;
+    constexpr int kKBytes = KT * KRowB, kVBytes = 2 * VBuf * 4;
+    constexpr int kMBytes = 4 * QW * 4;       // [key part][query]: maxima, then (S32) sums of P
+    constexpr int kBytes = kKBytes + kVBytes + kPBytes + kMBytes;
+    typedef WideLds<HD, FMT> L;
+    constexpr int kWideK = L::kKeys * sizeof(typename L::K), kWideV = 2 * sizeof(typename L::V);
+    constexpr int kWideBytes = QF32 ? 0 : kWideK + kWideV + 8 * sizeof(typename L::Ex);
+    __shared__ __align__(16) uint8_t lds[kBytes > kWideBytes ? kBytes : kWideBytes];
+    __shared__ uint32_t moved[2];             // a reference moves in this tile / the next
     uint8_t *const k_lds = lds;
-    uint32_t *const v_lds = reinterpret_cast<uint32_t *>(lds + L::kKBytes);
-    uint16_t *const p_lds = reinterpret_cast<uint16_t *>(lds + L::kKBytes + L::kVBytes);
-    float *const m_lds = reinterpret_cast<float *>(lds + L::kKBytes + L::kVBytes + L::kPBytes);
+    uint32_t *const v_lds = reinterpret_cast<uint32_t *>(lds + kKBytes);
+    uint16_t *const p_lds = reinterpret_cast<uint16_t *>(lds + kKBytes + kVBytes);
+    float *const m_lds = reinterpret_cast<float *>(lds + kKBytes + kVBytes + kPBytes);
     float *const l_lds = m_lds + 2 * QW;
     auto vt_at = [](int row, int col) { return row * VS + (row >> 4) * VPad + col; };
+
+    const int q0 = QF32 ? q0_host : (int)step[3];
+    if constexpr (!QF32)
+        if (q0 + n_tok <= (HD == 256 ? (n_tok > 64 ? 96 : 64) : n_tok > 32 ? 160 : 32)) {
+            prefill_wide<HD, FMT>(reinterpret_cast<typename L::K *>(lds),
+                                  reinterpret_cast<typename L::V *>(lds + kWideK),
+                                  reinterpret_cast<typename L::Ex *>(lds + kWideK + kWideV), nullptr,
+                                  nullptr, qv, q_scales, src, outv, n_tok, q0, n_q, n_kv, window, scale,
+                                  qtiles);
+            return;
+        }
 
     int bx = (int)blockIdx.x, by = (int)blockIdx.y;
     if (gridDim.y % 8 == 0) {  // XCD-aware order, as in attn_prefill_kernel
@@ -1578,42 +1598,6 @@ __device__ __forceinline__ void prefill_px(uint8_t *const lds, uint32_t *const m
         }
 }
 
-template <int HD>
-__global__ __launch_bounds__(512, 2) void attn_prefill_px_kernel(
-    const void *__restrict__ qv, const uint16_t *, KvSource src, void *__restrict__ outv, int n_tok,
-    int q0, const uint32_t *, int n_q, int n_kv, int window, float scale, int qtiles) {
-    __shared__ __align__(16) uint8_t lds[PxLds<HD>::kBytes];
-    __shared__ uint32_t moved[2];
-    prefill_px<HD, kPfQ8>(lds, moved, qv, src, outv, n_tok, q0, n_q, n_kv, window, scale, qtiles);
-}
-
-// The forms dispatched by name.  Their position, and with it the number of keys,
-// is known on the device only, so the choice between the two ways is made here.
-// us, prefill_wide / prefill_px as kernels of their own / here: head_dim 256, 16 /
-// 32 / 48 / 64 keys 6.5 / 7.8 / 6.7, 7.2 / 8.7 / 7.5, 10.1 / 10.0 / 10.3, 10.5 /
-// 11.0 / 10.9; 512, as many queries as keys, 64 / 128 / 160 / 192 15.4 / 16.4 / 15.6, 20.4 / 21.4 / 21.0,
-// 20.9 / 21.8 / 21.4, 26.4 / 26.8 / 26.6 (f16; Q8_0 the same within 0.3); 16
-// queries, 48 / 80 keys 11.0 / 11.0, 13.7 / 13.1.  LDS is the larger of both: one
-// workgroup per CU either way.
-template <int HD, int FMT>
-__global__ __launch_bounds__(512, 2) void attn_prefill_pages_kernel(
-    const void *__restrict__ qv, const uint16_t *, KvSource src, void *__restrict__ outv, int n_tok,
-    int, const uint32_t *__restrict__ step, int n_q, int n_kv, int window, float scale, int qtiles) {
-    typedef WideLds<HD, FMT> L;
-    constexpr int kKB = L::kKeys * (int)sizeof(typename L::K), kVB = 2 * (int)sizeof(typename L::V);
-    constexpr int kWide = kKB + kVB + 8 * (int)sizeof(typename L::Ex);
-    __shared__ __align__(16) uint8_t lds[kWide > PxLds<HD>::kBytes ? kWide : PxLds<HD>::kBytes];
-    __shared__ uint32_t moved[2];
-    const int q0 = (int)step[3];
-    if (q0 + n_tok <= (HD == 256 ? 64 : n_tok > 32 ? 160 : 32))
-        prefill_wide<HD, FMT>(reinterpret_cast<typename L::K *>(lds),
-                              reinterpret_cast<typename L::V *>(lds + kKB),
-                              reinterpret_cast<typename L::Ex *>(lds + kKB + kVB), nullptr, nullptr,
-                              qv, nullptr, src, outv, n_tok, q0, n_q, n_kv, window, scale, qtiles);
-    else
-        prefill_px<HD, FMT>(lds, moved, qv, src, outv, n_tok, q0, n_q, n_kv, window, scale, qtiles);
-}
-
 }  // namespace
 
 int launch_attn_prefill_ipv(hipStream_t st, const float *q, const int8_t *kq, const uint16_t *ks,
@@ -1668,21 +1652,25 @@ int launch_attn_prefill_q8(hipStream_t st, const float *q, const int8_t *kq, con
         const uint16_t *no_qs = nullptr;
         // Few keys in all: the wide kernel's shorter way through a single tile, with
         // the same bits.  us, wide / px: head_dim 256, 16 / 30 / 40 keys 8.0 / 8.9 /
-        // 12.0 against 9.2 / 10.2 / 11.4; 512, as many queries as keys, 20 / 100 /
+        // 12.0 against 9.2 / 10.2 / 11.4, and while px's last tile of 64 keys would be
+        // half empty (as many queries as keys, 64 / 80 / 96 / 100 / 160: 14.0 / 17.3 /
+        // 17.9 / 20.9 / 22.4 against 13.7 / 19.0 / 19.9 / 20.7 / 23.0); 512, as many queries as keys, 20 / 100 /
         // 320 / 500 / 700: 9.6 / 21.0 / 40.1 / 56.4 / 72.9 against 11.1 / 23.2 /
         // 42.1 / 56.7 / 72.7; 20 queries (px: a query tile without queries rests),
         // 100 / 200 / 320 keys 18.4 / 26.4 / 33.4 against 18.3 / 24.2 / 29.7.
         const int n_keys = q0 + n_tok;
-        const bool few_keys = n_keys <= (head_dim == 256 ? 32 : n_tok > 32 ? 512 : 96);
-#define SGQ_PF_Q8(...)                                                                           \
-    hipLaunchKernelGGL((__VA_ARGS__), grid, dim3(512), 0, st, q, no_qs, src, out, n_tok, q0, \
+        const bool few_keys =
+            head_dim == 256 ? n_keys <= 32 || (n_tok > 64 && n_keys <= 160 && (n_keys - 1) % 64 < 32)
+                            : n_keys <= (n_tok > 32 ? 512 : 96);
+#define SGQ_PF_Q8(KERNEL, HD)                                                                    \
+    hipLaunchKernelGGL((KERNEL<HD, kPfQ8>), grid, dim3(512), 0, st, q, no_qs, src, out, n_tok, q0, \
                        no_step, n_q, n_kv, window, scale, (int)grid.x)
         if (head_dim == 256) {
-            if (few_keys) SGQ_PF_Q8(attn_prefill_wide_kernel<256, kPfQ8>);
-            else SGQ_PF_Q8(attn_prefill_px_kernel<256>);
+            if (few_keys) SGQ_PF_Q8(attn_prefill_wide_kernel, 256);
+            else SGQ_PF_Q8(attn_prefill_px_kernel, 256);
         } else {
-            if (few_keys) SGQ_PF_Q8(attn_prefill_wide_kernel<512, kPfQ8>);
-            else SGQ_PF_Q8(attn_prefill_px_kernel<512>);
+            if (few_keys) SGQ_PF_Q8(attn_prefill_wide_kernel, 512);
+            else SGQ_PF_Q8(attn_prefill_px_kernel, 512);
         }
 #undef SGQ_PF_Q8
         SGQ_HIP(hipGetLastError());
@@ -1733,13 +1721,13 @@ int launch_attn_prefill_pages(hipStream_t st, int fmt, const void *q, const uint
     hipLaunchKernelGGL((KERNEL<HD, F>), grid, dim3(512), 0, st, q, q_scales, src, out, n_tok, 0,     \
                        step, n_q, n_kv, window, scale, qt)
     if (head_dim == 256) {
-        if (fmt == kPfQ8H) SGQ_PF_PAGES(attn_prefill_pages_kernel, 256, kPfQ8H);
-        else if (fmt == kPfF16) SGQ_PF_PAGES(attn_prefill_pages_kernel, 256, kPfF16);
+        if (fmt == kPfQ8H) SGQ_PF_PAGES(attn_prefill_px_kernel, 256, kPfQ8H);
+        else if (fmt == kPfF16) SGQ_PF_PAGES(attn_prefill_px_kernel, 256, kPfF16);
         else if (fmt == kPfIQ) SGQ_PF_PAGES(attn_prefill_wide_kernel, 256, kPfIQ);
         else SGQ_PF_PAGES(attn_prefill_wide_kernel, 256, kPfIPV);
     } else {
-        if (fmt == kPfQ8H) SGQ_PF_PAGES(attn_prefill_pages_kernel, 512, kPfQ8H);
-        else if (fmt == kPfF16) SGQ_PF_PAGES(attn_prefill_pages_kernel, 512, kPfF16);
+        if (fmt == kPfQ8H) SGQ_PF_PAGES(attn_prefill_px_kernel, 512, kPfQ8H);
+        else if (fmt == kPfF16) SGQ_PF_PAGES(attn_prefill_px_kernel, 512, kPfF16);
         else if (fmt == kPfIQ) SGQ_PF_PAGES(attn_prefill_wide_kernel, 512, kPfIQ);
         else SGQ_PF_PAGES(attn_prefill_wide_kernel, 512, kPfIPV);
     }

@@ -437,12 +437,12 @@ def test_prefill_int8_q_with_subnormal_scales(ctx, oracle, name, tiny):
 
 @pytest.mark.parametrize("name,q0,short,long_", [
     ("attn_prefill_sliding_ring", 0, 48, 80), ("attn_prefill_sliding_ring", 30, 32, 160),
-    ("attn_prefill_sliding", 0, 63, 66), ("attn_prefill_global_flash_sp", 0, 16, 48),
+    ("attn_prefill_sliding", 0, 64, 97), ("attn_prefill_sliding", 0, 96, 112), ("attn_prefill_global_flash_sp", 0, 16, 48),
     ("attn_prefill_global_flash_sp", 0, 160, 176), ("attn_prefill_global_flash_sp", 90, 64, 96),
     ("attn_prefill_global_flash_sp_q8", 0, 32, 192), ("attn_prefill_global_flash_sp_q8", 16, 16, 160)])
 def test_prefill_pages_rows_do_not_depend_on_the_chunk(ctx, oracle, name, q0, short, long_):
     """The kernel behind these names takes one way with few keys (64 at head_dim
-    256; at 512 160, or 32 for at most 32 queries) and another with more: the rows
+    256, 96 for more than 64 queries; at 512 160, or 32 for at most 32 queries) and another with more: the rows
     that a short and a long chunk share have the same bits, also where a reference
     maximum moves (later keys four times as large).  The short chunk is within the
     oracle's bars."""

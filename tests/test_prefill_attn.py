@@ -220,7 +220,7 @@ def test_attn_prefill_denominator_keeps_small_probabilities(ctx, oracle, hd, n_k
 
 
 @pytest.mark.parametrize("hd,q0,short,long_", [
-    (256, 0, 20, 150), (256, 0, 32, 33), (512, 0, 60, 600), (512, 60, 20, 470), (512, 0, 512, 513)])
+    (256, 0, 20, 150), (256, 0, 32, 33), (256, 0, 90, 97), (256, 0, 128, 160), (512, 0, 60, 600), (512, 60, 20, 470), (512, 0, 512, 513)])
 @pytest.mark.parametrize("grow", [1.0, 4.0])
 def test_attn_prefill_rows_do_not_depend_on_the_chunk(ctx, oracle, hd, q0, short, long_, grow):
     """Few keys take another kernel than many: the rows that a short and a long
