@@ -14,7 +14,7 @@
 //    logical K order of q4_0.rs:31-42 falls out with no shuffle.
 //  * Workgroup = 4 waves (2×2), tile 128×128, each wave 64×64 = 2×2 MFMA
 //    tiles.  A K-stage is 4 blocks (128 K): activations (int8) and weights
-//    (unpacked once per workgroup to int8 q-8 by the loading thread) go to
+//    (unpacked once per workgroup to int8 16·(q-8) by the loading thread) go to
 //    LDS, rows padded to 144 B so the 16-byte fragment reads of 8 lanes hit
 //    32 distinct banks.  Double-buffered: stage s+1's global loads are in
 //    flight while stage s computes; one barrier per stage.
@@ -26,7 +26,7 @@
 //    TOP/s, M = 4096 750 -> 786, with half the operand registers).  The VALU is
 //    left with one cvt and one FMA per output element and block, and that —
 //    not the MFMA — bounds the kernel: a wave64 VALU op holds its SIMD for 4
-//    cycles, and counters put VALU issue at 93% of the cycles (M = 4096,
+//    cycles, and counters put VALU issue at 88% of the cycles (M = 4096,
 //    K = 5376, N = 21504).  Every other VALU op of the loop therefore costs
 //    its share: with uniform pointers advanced by the scalar unit, one-op
 //    unpacks and the scale words moved up instead of selected, a stage takes
